@@ -30,11 +30,11 @@
 //                     lo part (two MFMAs per k-step), V^T via the
 //                     transposing LDS read ds_read_b64_tr_b16
 // The scores of tile i+1 are computed on MFMA while the exponentials of tile
-// i are formed.  Each row's softmax reference is fixed for the whole key
-// range (its first tile's max, subtracted inside the score MFMA by one extra
-// k-step), so the loop neither tracks maxima nor rescales; a row whose later
-// scores overflow or underflow the fp16 P shows it in its row sum, and its
-// wave runs again from the exact row maxima.
+// i are formed.  Each row's softmax reference is its first tile's max,
+// subtracted inside the score MFMA by one extra k-step, and stays until a
+// tile holds a score more than 15 log2 units above it (P's hi part is fp16):
+// the wave then raises the reference of such rows and scales what they have
+// summed so far, once per new peak.
 //
 // Query t at position start+t attends the window [pos-L+1, pos], L =
 // min(pos+1, max_seq) (mistral_ane_prefill.h:220-241); positions >= start come
@@ -583,22 +583,20 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     for (int st = 0; st < 8; ++st)
       ql[b][st] = *(lds_h8 *)(qs + (32 * b + col) * HD + 8 * ((2 * st + half) ^ swz(col)));
 
-  // Softmax reference per row, fixed for the whole key range of the wave:
-  // the max of the row's scores in its first tile (p <= 1 there), rounded to
-  // fp16 and subtracted inside the score MFMA by one extra k-step (a ones
-  // column in K against -m_ref in Q), so the loop neither subtracts nor
-  // tracks maxima and never rescales the accumulators.  P's hi part is fp16,
-  // so a later score more than ~16 (log2 units) above the reference
-  // overflows it, and a row whose scores all sit far below an unset reference
-  // underflows.  An underflowing row sums below 2^-8 (the fp32 row sum of the
-  // unrounded P).  A P that rounds to fp16 infinity (>= 65520) makes the row
-  // sum at least that and the row's accumulators non-finite (inf - inf from
-  // its hi and lo parts); the accumulators are only inspected when the sum
-  // is that large, so a long flat row with a large but finite sum costs one
-  // look at them, not a second pass.  A wave with such a row sweeps its tiles
-  // for the exact row maxima and runs once more with them as the reference.
+  // Softmax reference per row: the max of the row's scores in its first tile
+  // (p <= 1 there), rounded to fp16 hi + lo and subtracted inside the score
+  // MFMA by one extra k-step (a ones column in K against -m_ref in Q).  P's
+  // hi part is fp16, so a score may lie up to 16 above the reference: as long
+  // as none lies more than kRaise above it, the loop only compares each
+  // tile's scores with a per-row limit (raise_ref below does the rest), which
+  // sits in issue slots under the P.V MFMAs.  Model attention has such peaks
+  // (a few keys far above the first ones), and a second pass over the keys
+  // for rows that overflowed, the form before this one, ran 70.5 us instead
+  // of 38 at S 512 over 2048 keys with every 1024th key four times as large.
+  constexpr float kRaise = 15.0f;
   f16v o[NB][4];
   float m_ref[NB], l_run[NB];
+  float lim[NB];  // shifted scores above this raise the row's reference
   f16v s_cur[NB];
   h8 qx[NB];  // extra k-step B operand: -m_ref as fp16 hi, lo in elements 0, 1 of the half-0 lanes
 #pragma unroll
@@ -679,7 +677,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     for (int i = 2; i < 16; i += 2) m = fmaxf(m, fmaxf(s[i], s[i + 1]));
     return half_swap_max(m);
   };
-  // Unshifted scores of the tile in kt[buf] (first tile, max sweep).
+  // Unshifted scores of the wave's first tile.
   auto scores = [&](f16v (&sc)[NB], int buf, int kb) {
     h8 ka[8];
 #pragma unroll
@@ -694,6 +692,61 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     }
     qk_drain<NB>(sc);
     if (needs_mask(kb)) mask_tile(sc, kb);
+  };
+
+  auto max3 = [](float a, float b, float c) {
+    float d;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+  };
+  // Called when a (masked) tile's scores sc, shifted by the present
+  // references, may exceed a row's limit: rows that do get their max as the
+  // new reference (a row without one yet, whatever its max), and everything
+  // that carries the old one is scaled: the tile's scores, P of the tile
+  // before (pl, not yet in O), the row sum and O.
+  auto raise_ref = [&](f16v (&sc)[NB], h8 (&pl)[NB][4]) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const float m = block_max(sc[b]);
+      const bool up = m > lim[b], unset = m_ref[b] == -INFINITY;
+      const float old = unset ? 0.f : m_ref[b];
+      set_ref(b, up ? old + m : m_ref[b]);
+      const float d = (m_ref[b] == -INFINITY ? 0.f : m_ref[b]) - old;
+      const float f = unset ? 1.f : fast_exp2(-d);  // (an unset row has summed nothing)
+      if (up) lim[b] = kRaise;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sc[b][i] -= d;
+      l_run[b] *= f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u4 vh = __builtin_bit_cast(u4, pl[b][h]), vl = __builtin_bit_cast(u4, pl[b][2 + h]);
+        u4 nh, nl;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const unsigned eh = vh[k], el = vl[k];
+          const h2 ph = __builtin_bit_cast(h2, eh), pw = __builtin_bit_cast(h2, el);
+          unsigned hi, lo;
+          split_pair(((float)ph[0] + (float)pw[0]) * f, ((float)ph[1] + (float)pw[1]) * f, hi, lo);
+          nh[k] = hi;
+          nl[k] = lo;
+        }
+        pl[b][h] = __builtin_bit_cast(h8, nh);
+        pl[b][2 + h] = __builtin_bit_cast(h8, nl);
+      }
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[b][db][i] *= f;
+    }
+    // the accumulators were just written by the VALU, which the inline
+    // assembly MFMAs do not wait for
+    pv_drain_all(o);
+  };
+  auto any_above = [&](const float (&mx)[NB]) {
+    bool up = false;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) up = up || mx[b] > lim[b];
+    return __builtin_amdgcn_ballot_w64(up) != 0;
   };
 
   // One tile step, with P.V one tile behind the scores: P of tile it from
@@ -827,6 +880,20 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     // Window mask of tile it+1, only where it crosses a window edge.
     const int kbn = kb0 + kStride * (it + 1);
     if (needs_mask(kbn)) mask_tile(s_next, kbn);
+    if (it + 1 < g_count) {  // (a last step scores a buffer that holds no tile)
+      float mx[NB];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        mx[b] = s_next[b][0];
+#pragma unroll
+        for (int i = 1; i < 15; i += 2) mx[b] = max3(mx[b], s_next[b][i], s_next[b][i + 1]);
+        mx[b] = fmaxf(mx[b], s_next[b][15]);
+      }
+      if (any_above(mx)) {
+        pv_drain_all(o);
+        raise_ref(s_next, pb);
+      }
+    }
 #pragma unroll
     for (int b = 0; b < NB; ++b) s_cur[b] = s_next[b];
   };
@@ -921,6 +988,16 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     auto PVH = [&](int db, int b) {
       if (with_pv) mfma_pv2(o[b][db], vhi[db], p_in[b][1], p_in[b][3]);
     };
+    // Slice j (0 .. 7) of the new scores' maxima: four scores of block j / 4.
+    float mx[NB];
+    auto M = [&](int j) {
+      if (!with_qk) return;
+      const int b = j >> 2, e = 4 * (j & 3);
+      if (e == 0) mx[b] = s_out[b][0];
+      mx[b] = max3(mx[b], s_out[b][e], s_out[b][e + 1]);
+      mx[b] = max3(mx[b], s_out[b][e + 2], s_out[b][e + 3]);
+      asm volatile("" ::"v"(mx[b]));
+    };
     // slots 1-10: reference k-steps and k-steps 0-3; exponential slices 0-2
     REF(0); fence(); E(0, 0); fence();
     REF(1); fence(); E(0, 1); fence();
@@ -983,15 +1060,17 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     fence();
     // slots 27-34: P.V keys 16-31; V(it+1) goes into V(it-1)'s buffer once
     // every LDS read of the step is done
-    PVH(0, 0); fence(); E(6, 2); fence();
-    PVH(0, 1); fence(); E(6, 3); fence();
-    PVH(1, 0); keep(vhi[0]); fence(); E(7, 0); fence();
-    PVH(1, 1); fence(); E(7, 1); fence();
-    PVH(2, 0); keep(vhi[1]); fence(); E(7, 2); fence();
-    PVH(2, 1); fence(); E(7, 3); fence();
+    PVH(0, 0); fence(); E(6, 2); M(0); fence();
+    PVH(0, 1); fence(); E(6, 3); M(1); fence();
+    PVH(1, 0); keep(vhi[0]); fence(); E(7, 0); M(2); fence();
+    PVH(1, 1); fence(); E(7, 1); M(3); fence();
+    PVH(2, 0); keep(vhi[1]); fence(); E(7, 2); M(4); fence();
+    PVH(2, 1); fence(); E(7, 3); M(5); fence();
     PVH(3, 0);
     keep(vhi[2]);
     fence();
+    M(6);
+    M(7);
     if (it + 1 < g_count) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       MIA_LOAD_V_NEXT(it + 1, (it + 1) & 1);
@@ -1014,6 +1093,8 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     if (with_qk) {
       const int kbn = kb0 + kStride * (it + 1);
       if (needs_mask(kbn)) mask_tile(s_out, kbn);
+      // (a wave's only tile is followed by a scoring of no tile)
+      if (it + 1 < g_count && any_above(mx)) raise_ref(s_out, p_out);
     }
   };
   // O += P.V of the wave's last tile (its V in vt[(g_count-1)&1]) from P.
@@ -1043,140 +1124,97 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     pv_drain_all(o);
   };
 
-  for (int pass = 0; pass < 2; ++pass) {
-    if (pass == 1) {
-      // Exact row maxima over the wave's tiles, then the same pass again.
-      float mt[NB];
 #pragma unroll
-      for (int b = 0; b < NB; ++b) mt[b] = -INFINITY;
-      for (int i = 0; i < g_count; ++i) {
-        MIA_LOAD_K(i, 0);
-        wait_vmcnt<0>();
-        f16v sc[NB];
-        scores(sc, 0, kb0 + kStride * i);
+  for (int b = 0; b < NB; ++b) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) mt[b] = fmaxf(mt[b], block_max(sc[b]));
-      }
+    for (int db = 0; db < 4; ++db) mfma_zero(o[b][db], zero8);
+    l_run[b] = 0.f;
 #pragma unroll
-      for (int b = 0; b < NB; ++b) set_ref(b, mt[b]);
-      issue_first_tiles();
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-#pragma unroll
-      for (int db = 0; db < 4; ++db) mfma_zero(o[b][db], zero8);
-      l_run[b] = 0.f;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s_cur[b][i] = -INFINITY;
-    }
-    // The first tile's scores set the reference (first pass) and are
-    // shifted by it.
-    if (g_count > 0) {
-      if (g_count > 1) wait_vmcnt<16>();  // K1 and V0 may be pending
-      else wait_vmcnt<8>();
-      scores(s_cur, 0, kb0);
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        if (pass == 0) set_ref(b, block_max(s_cur[b]));
-        const float sh = m_ref[b] == -INFINITY ? 0.f : m_ref[b];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s_cur[b][i] -= sh;
-      }
-    } else {
-#pragma unroll
-      for (int b = 0; b < NB; ++b) set_ref(b, -INFINITY);
-    }
-
-    // Loads are issued in the order K0 K1 V0 | K2 V1 | K3 V2 | ... (step it
-    // issues K(it+2), then V(it+1)).  Step it needs K(it+1) and V(it-1): only
-    // V(it), the last load issued, may still be pending.
-    if constexpr (NB == 2) {
-      // Step it exponentiates tile it and scores tile it+1; the last step
-      // (it = g_count - 1) scores nothing.
-      using T = std::true_type;
-      using F = std::false_type;
-      f16v s_alt[NB];
-      h8 p_a[NB][4], p_b[NB][4];
-      if (g_count > 0) {
-        wait_vmcnt<8>();
-        step2(0, F{}, T{}, s_cur, s_alt, p_a, p_b);  // P(0) -> p_b
-      }
-      int it = 1;
-      for (; it + 2 < g_count; it += 2) {
-        wait_vmcnt<8>();
-        step2(it, T{}, T{}, s_alt, s_cur, p_b, p_a);
-        wait_vmcnt<8>();
-        step2(it + 1, T{}, T{}, s_cur, s_alt, p_a, p_b);
-      }
-      if (it + 1 < g_count) {  // it = g_count - 2: one more scoring step
-        wait_vmcnt<8>();
-        step2(it, T{}, T{}, s_alt, s_cur, p_b, p_a);
-        ++it;
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {  // into the registers the last step reads
-          s_alt[b] = s_cur[b];
-#pragma unroll
-          for (int h = 0; h < 4; ++h) p_b[b][h] = p_a[b][h];
-        }
-      }
-      if (it < g_count) {  // it = g_count - 1: the last step
-        wait_vmcnt<8>();
-        step2(it, T{}, F{}, s_alt, s_cur, p_b, p_a);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {  // P of the last tile where last_pv_of reads it
-#pragma unroll
-          for (int h = 0; h < 4; ++h) p_b[b][h] = p_a[b][h];
-        }
-      }
-      if (g_count > 0) {
-        wait_vmcnt<0>();
-        last_pv_of(p_b);
-      }
-    } else {
-      if (g_count > 0) {
-        wait_vmcnt<8>();
-        step(0, std::false_type{});
-      }
-      for (int it = 1; it < g_count; ++it) {
-        wait_vmcnt<8>();
-        step(it, std::true_type{});
-      }
-      if (g_count > 0) {
-        wait_vmcnt<0>();
-        last_pv();
-      }
-    }
-    // Row sums: an underflow (< 2^-8 with keys in range, or not finite) means
-    // the reference did not suit the row; so does an fp16 overflow of some P,
-    // possible only where the sum reaches 65504 and then visible as a
-    // non-finite accumulator of the row.
-    bool bad = false, large = false;
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const float lt = half_swap_sum(l_run[b]);
-      l_run[b] = lt;
-      bad = bad || (has_keys[b] && !(lt >= 0.00390625f));
-      large = large || (has_keys[b] && !(lt < 65504.0f));
-    }
-    if (pass == 0 && __builtin_amdgcn_ballot_w64(large) != 0) {
-      pv_drain<NB>(o);
-      bool nonfinite = false;
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        // a sum of the row's accumulators is non-finite iff one of them is
-        // (at magnitudes far below fp32's range)
-        float t = 0.f;
-#pragma unroll
-        for (int db = 0; db < 4; ++db)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) t += o[b][db][i];
-        t = half_swap_sum(t);
-        nonfinite = nonfinite || (has_keys[b] && !__builtin_isfinite(t));
-      }
-      bad = bad || nonfinite;
-    }
-    if (pass == 1 || __builtin_amdgcn_ballot_w64(bad) == 0) break;
+    for (int i = 0; i < 16; ++i) s_cur[b][i] = -INFINITY;
   }
+  // The first tile's scores set the reference and are shifted by it.
+  if (g_count > 0) {
+    if (g_count > 1) wait_vmcnt<16>();  // K1 and V0 may be pending
+    else wait_vmcnt<8>();
+    scores(s_cur, 0, kb0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      set_ref(b, block_max(s_cur[b]));
+      const float sh = m_ref[b] == -INFINITY ? 0.f : m_ref[b];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s_cur[b][i] -= sh;
+    }
+  } else {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) set_ref(b, -INFINITY);
+  }
+  // A row that has keys later but none in the first tile takes its
+  // reference from the first tile that has some.
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    lim[b] = !has_keys[b] ? INFINITY : (m_ref[b] == -INFINITY ? -INFINITY : kRaise);
+
+  // Loads are issued in the order K0 K1 V0 | K2 V1 | K3 V2 | ... (step it
+  // issues K(it+2), then V(it+1)).  Step it needs K(it+1) and V(it-1): only
+  // V(it), the last load issued, may still be pending.
+  if constexpr (NB == 2) {
+    // Step it exponentiates tile it and scores tile it+1; the last step
+    // (it = g_count - 1) scores nothing.
+    using T = std::true_type;
+    using F = std::false_type;
+    f16v s_alt[NB];
+    h8 p_a[NB][4], p_b[NB][4];
+    if (g_count > 0) {
+      wait_vmcnt<8>();
+      step2(0, F{}, T{}, s_cur, s_alt, p_a, p_b);  // P(0) -> p_b
+    }
+    int it = 1;
+    for (; it + 2 < g_count; it += 2) {
+      wait_vmcnt<8>();
+      step2(it, T{}, T{}, s_alt, s_cur, p_b, p_a);
+      wait_vmcnt<8>();
+      step2(it + 1, T{}, T{}, s_cur, s_alt, p_a, p_b);
+    }
+    if (it + 1 < g_count) {  // it = g_count - 2: one more scoring step
+      wait_vmcnt<8>();
+      step2(it, T{}, T{}, s_alt, s_cur, p_b, p_a);
+      ++it;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {  // into the registers the last step reads
+        s_alt[b] = s_cur[b];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) p_b[b][h] = p_a[b][h];
+      }
+    }
+    if (it < g_count) {  // it = g_count - 1: the last step
+      wait_vmcnt<8>();
+      step2(it, T{}, F{}, s_alt, s_cur, p_b, p_a);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {  // P of the last tile where last_pv_of reads it
+#pragma unroll
+        for (int h = 0; h < 4; ++h) p_b[b][h] = p_a[b][h];
+      }
+    }
+    if (g_count > 0) {
+      wait_vmcnt<0>();
+      last_pv_of(p_b);
+    }
+  } else {
+    if (g_count > 0) {
+      wait_vmcnt<8>();
+      step(0, std::false_type{});
+    }
+    for (int it = 1; it < g_count; ++it) {
+      wait_vmcnt<8>();
+      step(it, std::true_type{});
+    }
+    if (g_count > 0) {
+      wait_vmcnt<0>();
+      last_pv();
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < NB; ++b) l_run[b] = half_swap_sum(l_run[b]);
 #undef MIA_LOAD_FAST
 #undef MIA_LOAD_K
 #undef MIA_LOAD_V

@@ -245,3 +245,29 @@ def test_verify_step_65536_peaked_large_v():
         exact[t] = D.gqa_decode_f64(Qr[t], rk, rv, 32, 8, 128, M, start + t)
     assert np.abs(exact).max() > 16.0
     _check_vs_exact_and_oracle(out, exact, ref, "verify 65536 peaked large V")
+
+
+@pytest.mark.parametrize("M,start,S,peaks", [
+    (4096, 1536, 64, (33, 700, 1599)),   # 64-row tiles: second tile, mid-range, the last key
+    (4096, 0, 70, (31, 32, 69)),         # rows whose waves have no keys in their first tile
+    (4096, 500, 8, (64, 507)),           # 32-row tiles
+    (300, 1000, 40, (5, 250)),           # wrapped windows (slots): rows that start mid-tile
+    (300, 1000, 8, (5, 104, 250)),
+])
+def test_attention_batch_peaks_raise_the_reference(M, start, S, peaks):
+    # A few keys 16 times as large: scores reach +-70 log2 units, so rows
+    # raise their softmax reference at those tiles (and only some rows of a
+    # wave do).  Against float64, with V ~ 8 N(0,1): what was summed before a
+    # peak must be scaled with it, at the precision of the other rows.
+    G.say(f"attention_batch peaks M={M} start={start} S={S} at {peaks}")
+    g = D.rng(300 + S + M)
+    kc, vc = _peaked_large_v(g, M, start + S, sigma=1.0)
+    for p in peaks:
+        kc[p] = D.to_f16_bits(16.0 * D.f16_bits_to_f32(kc[p]))
+    Q = D.normal(g, (S, 4096))
+    out = G.attention_batch(Q, kc, vc, M, start, S)
+    exact = np.empty((S, 4096))
+    for t in range(S):  # the ring as it stands holds the positions up to start + S - 1
+        n = min(start + t + 1, M)
+        exact[t] = D.gqa_decode_f64(Q[t], kc[:n], vc[:n], 32, 8, 128, n, n - 1)
+    D.check_close(out, exact, what=f"peaks M={M} start={start} S={S}")
