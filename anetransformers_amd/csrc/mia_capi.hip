@@ -488,8 +488,8 @@ int flash_impl(DevCtx *c, const float *Q, const float *rope_cs, const uint16_t *
                int n_kv, int max_seq, int start_pos, int S, hipStream_t s, bool commit = false) {
   mia::FlashParams p{};
   int rt = 0;
-  mia::flash_plan(S, n_kv, kG, start_pos, max_seq, c->num_cus, &p.n_rtiles, &p.nsplit,
-                  &p.split_keys, &rt);
+  mia::flash_plan(S, n_kv, kG, start_pos, max_seq, kst != nullptr, c->num_cus, &p.n_rtiles,
+                  &p.nsplit, &p.split_keys, &rt);
   p.Q = Q;
   p.rope_cs = rope_cs;
   p.kc = reinterpret_cast<const _Float16 *>(k_layer);

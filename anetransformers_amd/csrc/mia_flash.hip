@@ -334,13 +334,16 @@ __device__ __forceinline__ void pv_drain_all(f16v (&o)[NB][4]) {
 __device__ __forceinline__ float half_swap_max(float m) { return fmaxf(m, __shfl_xor(m, 32)); }
 __device__ __forceinline__ float half_swap_sum(float x) { return x + __shfl_xor(x, 32); }
 
-// FAST: every key range starts at key 0 of an unwrapped ring with no staged
-// rows and holds at least one whole tile (flash_fast_ok), so every tile's 32
-// rows are 32 consecutive ring slots: all loads take the uniform-base form,
-// and the last, partial tile of a range is loaded as the 32 keys ending at
-// the range end, with the keys before the tile's own start masked.  The
-// generic kernel handles wrapped windows, staged rows and short ranges with
-// per-lane addresses on the tiles that need them.
+// FAST: no staged rows.  The keys are then the ring's slots as they stand:
+// the window of position p, min(p + 1, max_seq) positions, is the slots 0 ..
+// min(p, max_seq - 1) whatever the ring's start, and the order of a softmax
+// does not matter, so "keys" are slots here, every window starts at key 0 and
+// no tile wraps.  Every tile's 32 rows are 32 consecutive slots: all loads take
+// the uniform-base form, and the last, partial tile of a range is loaded as the
+// 32 keys ending at the range end, with the keys before the tile's own start
+// masked (a range that ends before key 32 repeats its last key instead).  The
+// generic kernel has wrapped windows next to staged rows, with per-lane
+// addresses on the tiles that need them.
 template <int NB, bool FAST>
 __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   using L = Lay<NB>;
@@ -364,8 +367,9 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   // Key range of the workgroup (one split), then of this wave.
   const int tq0 = row0 >> 2;
   const int tq1 = min(tq0 + RT / 4 - 1, p.S - 1);
-  const int klo = window_lo(p.start_pos + tq0, p.max_seq);
-  const int khi = p.start_pos + tq1;
+  const int klo = FAST ? 0 : window_lo(p.start_pos + tq0, p.max_seq);
+  const int kcap = FAST ? p.max_seq - 1 : INT_MAX;  // the last key there is
+  const int khi = min(p.start_pos + tq1, kcap);
   const int ks = klo + split * p.split_keys;
   const int ke = min(ks + p.split_keys, khi + 1);
   const int nt = ke > ks ? (ke - ks + kKT - 1) / kKT : 0;
@@ -387,13 +391,13 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     const int t = (row0 + 32 * b + col) >> 2;
     valid[b] = t < p.S;
     const int pos_t = p.start_pos + (valid[b] ? t : p.S - 1);
-    lo_t[b] = window_lo(pos_t, p.max_seq);
-    hi_t[b] = pos_t;
+    lo_t[b] = FAST ? 0 : window_lo(pos_t, p.max_seq);
+    hi_t[b] = min(pos_t, kcap);
     const int ts0 = (row0 + 32 * b) >> 2;
     const int ts1 = (row0 + 32 * b + 31) >> 2;
     bfull[b] = ts1 < p.S;
-    lo_max[b] = window_lo(p.start_pos + min(ts1, p.S - 1), p.max_seq);
-    hi_min[b] = p.start_pos + ts0;
+    lo_max[b] = FAST ? 0 : window_lo(p.start_pos + min(ts1, p.S - 1), p.max_seq);
+    hi_min[b] = min(p.start_pos + ts0, kcap);
   }
   // Does the lane's row of block b have a key in this wave's range?
   bool has_keys[NB];
@@ -436,7 +440,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   const _Float16 *const kst = p.kstage, *const vst = p.vstage;
   auto tile_slot = [&](int i) { return (kb0 + kStride * i) % p.max_seq; };
   // FAST: first key (= ring slot) of the 32 rows loaded for tile i.
-  auto fast_slot = [&](int i) { return min(kb0 + kStride * i, ke - kKT); };
+  auto fast_slot = [&](int i) { return max(min(kb0 + kStride * i, ke - kKT), 0); };
   // Ring slots of the next K and V tiles to load, advanced by one stride per
   // load (no division in the tile loop).
   int kslot = 0, vslot = 0;
@@ -487,6 +491,14 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   } while (0)
   // K0, K1, then V0: V(i) is first needed one step after K(i+1).
   auto issue_first_tiles = [&]() {
+    if (FAST && ke < kKT) {
+      // a range shorter than a tile is one wave's only tile
+      if (g_count > 0) {
+        load_tile(kc, nullptr, 0, 0, ke, 0, INT_MAX, kv_dim, kvh * HD, boff, lane, kt_a[0]);
+        load_tile(vc, nullptr, 0, 0, ke, 0, INT_MAX, kv_dim, kvh * HD, boff, lane, vt_a[0]);
+      }
+      return;
+    }
     if (g_count > 0) MIA_LOAD_K(0, 0);
     if (g_count > 1) MIA_LOAD_K(1, 1);
     if (g_count > 0) MIA_LOAD_V(0, 0);
@@ -596,7 +608,6 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   constexpr float kRaise = 15.0f;
   f16v o[NB][4];
   float m_ref[NB], l_run[NB];
-  float lim[NB];  // shifted scores above this raise the row's reference
   f16v s_cur[NB];
   h8 qx[NB];  // extra k-step B operand: -m_ref as fp16 hi, lo in elements 0, 1 of the half-0 lanes
 #pragma unroll
@@ -658,7 +669,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     for (int i = 0; i < 16; ++i) s[i] = (i >> 2) * 8 + (i & 3) <= hr ? s[i] : -INFINITY;
   };
   auto mask_tile = [&](f16v (&sc)[NB], int kb) {
-    const int kbl = FAST ? min(kb, ke - kKT) : kb;
+    const int kbl = FAST ? max(min(kb, ke - kKT), 0) : kb;
     bool lo_free = kbl == kb;
 #pragma unroll
     for (int b = 0; b < NB; ++b) lo_free = lo_free && kb >= lo_max[b];
@@ -708,12 +719,11 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const float m = block_max(sc[b]);
-      const bool up = m > lim[b], unset = m_ref[b] == -INFINITY;
+      const bool unset = m_ref[b] == -INFINITY, up = m > (unset ? -INFINITY : kRaise);
       const float old = unset ? 0.f : m_ref[b];
       set_ref(b, up ? old + m : m_ref[b]);
       const float d = (m_ref[b] == -INFINITY ? 0.f : m_ref[b]) - old;
       const float f = unset ? 1.f : fast_exp2(-d);  // (an unset row has summed nothing)
-      if (up) lim[b] = kRaise;
 #pragma unroll
       for (int i = 0; i < 16; ++i) sc[b][i] -= d;
       l_run[b] *= f;
@@ -745,7 +755,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   auto any_above = [&](const float (&mx)[NB]) {
     bool up = false;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) up = up || mx[b] > lim[b];
+    for (int b = 0; b < NB; ++b) up = up || mx[b] > (m_ref[b] == -INFINITY ? -INFINITY : kRaise);
     return __builtin_amdgcn_ballot_w64(up) != 0;
   };
 
@@ -1148,16 +1158,17 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) set_ref(b, -INFINITY);
   }
-  // A row that has keys later but none in the first tile takes its
-  // reference from the first tile that has some.
+  // A row that has keys later but none in the first tile takes its reference
+  // from the first tile that has some; a row without any keeps 0 (its scores
+  // are all masked, and the merge gives it no weight).
 #pragma unroll
   for (int b = 0; b < NB; ++b)
-    lim[b] = !has_keys[b] ? INFINITY : (m_ref[b] == -INFINITY ? -INFINITY : kRaise);
+    if (!has_keys[b]) set_ref(b, 0.f);
 
   // Loads are issued in the order K0 K1 V0 | K2 V1 | K3 V2 | ... (step it
   // issues K(it+2), then V(it+1)).  Step it needs K(it+1) and V(it-1): only
   // V(it), the last load issued, may still be pending.
-  if constexpr (NB == 2) {
+  if constexpr (NB == 2 && FAST) {
     // Step it exponentiates tile it and scores tile it+1; the last step
     // (it = g_count - 1) scores nothing.
     using T = std::true_type;
@@ -1399,22 +1410,11 @@ hipError_t set_lds_limit() {
 
 int rows_per_tile(int S) { return S * 4 <= 32 ? 32 : 64; }
 
-// The FAST kernel's conditions: no staged rows, no key split, no window
-// reaching past the ring's end (every row's window starts at key 0 and no
-// tile wraps), and every workgroup's key range at least one tile long (the
-// shortest is the first row tile's, start_pos + its query count).
-bool flash_fast_ok(const FlashParams &p) {
-  const int first_rows = rows_per_tile(p.S) / 4;
-  return p.kstage == nullptr && p.vstage == nullptr && p.nsplit == 1 &&
-         (long)p.start_pos + p.S <= (long)p.max_seq &&
-         (long)p.start_pos + (p.S < first_rows ? p.S : first_rows) >= kKT;
-}
-
 template <int NB>
 hipError_t launch_variant(const FlashParams &p, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
   using L = Lay<NB>;
   dim3 grid(p.n_kv * p.n_rtiles * p.nsplit);
-  if (flash_fast_ok(p))
+  if (p.kstage == nullptr && p.vstage == nullptr)
     hipExtLaunchKernelGGL((flash_kernel<NB, true>), grid, dim3(256), L::kBytes, s, ev0, ev1, 0, p);
   else
     hipExtLaunchKernelGGL((flash_kernel<NB, false>), grid, dim3(256), L::kBytes, s, ev0, ev1, 0,
@@ -1438,9 +1438,13 @@ size_t flash_scratch_bytes(int n_kv, int n_rtiles, int nsplit, int rows_per_tile
 // Few rows (S*G <= 32, e.g. speculative verify): one 32-row block, key splits
 // over workgroups until about target_wgs workgroups.  Otherwise (prefill):
 // 64-row tiles, no split unless the row tiles alone leave the device mostly
-// idle.  Every wave of a split keeps at least 4 tiles of 32 keys.
-void flash_plan(int S, int n_kv, int G, int start_pos, int max_seq, int target_wgs, int *n_rtiles,
-                int *nsplit, int *split_keys, int *rows_per_tile_out) {
+// idle.  Every wave of a split keeps at least one tile of 32 keys, and ranges of
+// fewer than four such splits stay whole (eight drafts after 250 keys, two
+// splits: 56 against 50 us for four layers; after 1000 keys, seven splits: 56.5
+// against 69.8 unsplit, and 65.1 with at least two tiles a wave).
+// Without staged rows keys are slots (flash_kernel).
+void flash_plan(int S, int n_kv, int G, int start_pos, int max_seq, bool staged, int target_wgs,
+                int *n_rtiles, int *nsplit, int *split_keys, int *rows_per_tile_out) {
   const int rt = rows_per_tile(S);
   const int ntiles = (S * G + rt - 1) / rt;
   long maxkeys = 0;
@@ -1449,13 +1453,15 @@ void flash_plan(int S, int n_kv, int G, int start_pos, int max_seq, int target_w
     int t1 = ((ti + 1) * rt - 1) / G;
     if (t1 > S - 1) t1 = S - 1;
     long p0 = (long)start_pos + t0;
-    long lo = p0 + 1 > max_seq ? p0 + 1 - max_seq : 0;
+    long lo = staged && p0 + 1 > max_seq ? p0 + 1 - max_seq : 0;
     long hi = (long)start_pos + t1;
+    if (!staged && hi > max_seq - 1) hi = max_seq - 1;
     if (hi - lo + 1 > maxkeys) maxkeys = hi - lo + 1;
   }
   long want = (long)target_wgs / ((long)n_kv * ntiles);
   if (want < 1) want = 1;
-  long max_split = maxkeys / (4L * kWaves * kKT);
+  long max_split = maxkeys / (kWaves * kKT);
+  if (max_split < 4) max_split = 1;
   if (max_split > kMergeSplitsPerThread * 32) max_split = kMergeSplitsPerThread * 32;
   if (want > max_split) want = max_split > 0 ? max_split : 1;
   long sk = (maxkeys + want - 1) / want;

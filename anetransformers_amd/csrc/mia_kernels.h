@@ -76,7 +76,7 @@ size_t flash_scratch_bytes(int n_kv, int n_rtiles, int nsplit, int rows_per_tile
 // ev0/ev1 (may be null) are stamped at the kernel's start and end.
 hipError_t launch_flash(const FlashParams &p, int G, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1);
 hipError_t launch_flash_merge(const FlashParams &p, hipStream_t s);
-void flash_plan(int S, int n_kv, int G, int start_pos, int max_seq, int target_wgs,
+void flash_plan(int S, int n_kv, int G, int start_pos, int max_seq, bool staged, int target_wgs,
                 int *n_rtiles, int *nsplit, int *split_keys, int *rows_per_tile);
 
 // Elementwise helpers.

@@ -271,3 +271,27 @@ def test_attention_batch_peaks_raise_the_reference(M, start, S, peaks):
         n = min(start + t + 1, M)
         exact[t] = D.gqa_decode_f64(Q[t], kc[:n], vc[:n], 32, 8, 128, n, n - 1)
     D.check_close(out, exact, what=f"peaks M={M} start={start} S={S}")
+
+
+@pytest.mark.parametrize("M,start,S", [
+    (8192, 0, 1), (8192, 0, 17), (8192, 30, 2),   # row tiles with fewer keys than a tile
+    (24, 100, 5),                                 # a ring smaller than a tile
+    (300, 290, 40),                               # a chunk that wraps: windows of 291 .. 300 slots
+    (300, 1000, 70), (1024, 5000, 16),            # wrapped, whole ring; split over workgroups
+    (4096, 900, 16), (4096, 505, 8),              # the shortest ranges that are split
+])
+def test_attention_batch_ring_in_slot_order(M, start, S):
+    # Attention over the ring as it stands walks slots 0 .. min(pos, M - 1);
+    # slots no window reaches hold NaN and must not be read into a product.
+    G.say(f"attention_batch slot order M={M} start={start} S={S}")
+    g = D.rng(M + start + S)
+    filled = min(start + S, M)
+    kc, vc = D.ring(g, M, filled=filled)
+    kc[filled:], vc[filled:] = 0x7E00, 0x7E00
+    Q = D.normal(g, (S, 4096))
+    out = G.attention_batch(Q, kc, vc, M, start, S)
+    exact = np.empty((S, 4096))
+    for t in range(S):
+        n = min(start + t + 1, M)
+        exact[t] = D.gqa_decode_f64(Q[t], kc[:n], vc[:n], 32, 8, 128, n, n - 1)
+    D.check_close(out, exact, what=f"slot order M={M} start={start} S={S}")
