@@ -33,7 +33,7 @@ constexpr int kMaxSeq = 1 << 22;  // ring capacity limit; in-layer offsets are 6
 // token takes its slot by scanning them (S^2 / 2 reads); longer chunks use a
 // per-slot area instead (one more launch, linear in S).
 constexpr int kChunkScanMax = 64;
-// The fp16 GEMMs of the weight types other than Q4_0 (hipBLASLt): workspace
+// The K and V projections of layers of other weight types (hipBLASLt): workspace
 // size, algorithms timed on a shape's first call, shapes remembered.
 constexpr size_t kLtWorkspace = size_t(64) << 20;
 constexpr int kLtCandidates = 4;
@@ -63,15 +63,15 @@ struct DevCtx {
   size_t split_work_bytes = 0;
   int *owner = nullptr;  // long chunks of mia_attention_chunk: last token per ring slot, -1 at rest
   int owner_slots = 0;
-  // Weight types other than Q4_0 in the GEMM: the weights' fp16 planes and
-  // the partial products, multiplied by hipBLASLt (handle and workspace
-  // created on first use, the algorithm of each GEMM shape picked on its
-  // first call: lt_gemm).
-  float *wbuf = nullptr;
-  size_t wbuf_bytes = 0;
+  // hipBLASLt: handle and workspace created on first use, the algorithm of
+  // each shape picked on its first call (lt_gemm), operands and products
   hipblasLtHandle_t lt = nullptr;
   void *lt_ws = nullptr;
   std::vector<LtPick> lt_picks;
+  void *lt_buf = nullptr;
+  size_t lt_buf_bytes = 0;
+  void *wbuf = nullptr;  // a GEMM's Q6_K weights regrouped, or its F32 weights as fp16 planes
+  size_t wbuf_bytes = 0;
   void *dl_work = nullptr;  // mia_decode_layer's vectors
   size_t dl_work_bytes = 0;
   // Opt-in kernel timing: an event pair around the main kernel of each call
@@ -201,7 +201,7 @@ int ensure_wbuf(DevCtx *c, size_t bytes) {
     if (c->wbuf) HIP_TRY(hipFree(c->wbuf));
     c->wbuf = nullptr;
     c->wbuf_bytes = 0;
-    HIP_TRY(hipMalloc((void **)&c->wbuf, bytes));
+    HIP_TRY(hipMalloc(&c->wbuf, bytes));
     c->wbuf_bytes = bytes;
   }
   return MIA_OK;
@@ -215,6 +215,18 @@ int ensure_dl_work(DevCtx *c, size_t bytes) {
     c->dl_work_bytes = 0;
     HIP_TRY(hipMalloc(&c->dl_work, bytes));
     c->dl_work_bytes = bytes;
+  }
+  return MIA_OK;
+}
+
+int ensure_lt_buf(DevCtx *c, size_t bytes) {
+  if (bytes > c->lt_buf_bytes) {
+    HIP_TRY(hipDeviceSynchronize());
+    if (c->lt_buf) HIP_TRY(hipFree(c->lt_buf));
+    c->lt_buf = nullptr;
+    c->lt_buf_bytes = 0;
+    HIP_TRY(hipMalloc(&c->lt_buf, bytes));
+    c->lt_buf_bytes = bytes;
   }
   return MIA_OK;
 }
@@ -565,16 +577,33 @@ int q4_impl(const void *Wq, const void *Wk, const void *Wv, const void *x_q8, co
 
 }  // namespace
 
-// Q4_0 GEMM over up to three stacked matrices (see GemmParams).
-int gemm_impl(DevCtx *c, const void *W0, const void *W1, const void *W2, int rows0, int rows1,
-              int rows2, const float *X, int K, int S, float *y0, float *y1, float *y2, int mode,
-              hipStream_t s, bool reuse_split = false, const _Float16 *planes = nullptr,
-              _Float16 *out_planes = nullptr, bool packed = false) {
-  // X [S][K] as fp16 hi + lo planes in split_work; reuse_split: the planes of
-  // the input are already there (written by the call before on this stream,
-  // or by the RMSNorm that produced them), and X is not read.
-  // planes: the input's planes given by the caller ([S][K] hi, then lo).
-  // out_planes (kGemmSiluMul): the result as planes there instead of in y0.
+static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// The GEMM's packed form of a matrix of a type other than Q4_0: the fp16 hi
+// plane [N][K], then for Q6_K / F32 the lo plane [N][K] and the row scales [N]
+// fp32, each at a 256-byte aligned offset (launch_typed_split's output).
+static size_t typed_planes_bytes(int type, int N, int K) {
+  const bool lo = !mia::typed_is_f16_exact(type);
+  const size_t bw = al256((size_t)N * K * 2);
+  return lo ? 2 * bw + al256((size_t)N * 4) : bw;
+}
+
+// Types whose matrices go through the GEMM one at a time, as hi + lo planes.
+static bool gemm_two_planes(int type) { return type == MIA_TYPE_Q6_K || type == MIA_TYPE_F32; }
+
+// The GEMM over up to three stacked matrices of one type (see GemmParams), as
+// the file holds them or (packed) in mia_gemm_pack's form.  X [S][K] goes
+// into split_work as fp16 hi + lo planes; reuse_split: the planes of the
+// input are already there (written by the call before on this stream, or by
+// the RMSNorm that produced them), and X is not read; planes: the input's
+// planes given by the caller ([S][K] hi, then lo).  out_planes (kGemmSwiGlu,
+// W0 the gate and W1 the up matrix): the result as planes [S][rows0] there.
+// plain_split: gemm_plan's.
+int gemm_impl(DevCtx *c, int type, const void *W0, const void *W1, const void *W2, int rows0,
+              int rows1, int rows2, const float *X, int K, int S, float *y0, float *y1, float *y2,
+              int mode, hipStream_t s, bool packed, bool reuse_split = false,
+              const _Float16 *planes = nullptr, _Float16 *out_planes = nullptr,
+              bool plain_split = false) {
   const size_t n = (size_t)S * K;
   const bool have = reuse_split || planes != nullptr;
   if (!have) {
@@ -591,7 +620,7 @@ int gemm_impl(DevCtx *c, const void *W0, const void *W1, const void *W2, int row
   p.alo = alo;
   if (out_planes != nullptr) {
     p.ohi = out_planes;
-    p.olo = out_planes + (size_t)S * (rows0 + rows1 + rows2);
+    p.olo = out_planes + (size_t)S * rows0;
   }
   p.w0 = reinterpret_cast<const uint8_t *>(W0);
   p.w1 = reinterpret_cast<const uint8_t *>(W1);
@@ -604,15 +633,74 @@ int gemm_impl(DevCtx *c, const void *W0, const void *W1, const void *W2, int row
   p.y0 = y0;
   p.y1 = y1;
   p.y2 = y2;
-  p.packed = packed ? 1 : 0;
-  p.ksplit = mia::gemm_pick_ksplit(p.N, K, S, c->num_cus);
+  if (type == MIA_TYPE_Q4_0) {
+    p.src = packed ? mia::kGemmQ40Tile : mia::kGemmQ40;
+  } else if (type == MIA_TYPE_Q4_K && !packed) {
+    p.src = mia::kGemmQ4K;
+  } else if (!gemm_two_planes(type)) {
+    p.src = mia::kGemmF16;
+  } else if (type == MIA_TYPE_Q6_K && !packed) {
+    p.src = mia::kGemmQ6K;
+    const size_t bw = al256((size_t)rows0 * K);
+    if (int rc = ensure_wbuf(c, bw + (size_t)rows0 * sizeof(float))) return rc;
+    uint8_t *w = reinterpret_cast<uint8_t *>(c->wbuf);
+    float *rs = reinterpret_cast<float *>(w + bw);
+    HIP_TRY(mia::launch_q6k_regroup(W0, w, rs, rows0, K, s));
+    p.w0 = w;
+    p.row_scale = rs;
+  } else {
+    p.src = mia::kGemmF16x2;
+    const size_t bw = al256((size_t)rows0 * K * 2);
+    if (!packed) {
+      if (int rc = ensure_wbuf(c, typed_planes_bytes(type, rows0, K))) return rc;
+      char *w = reinterpret_cast<char *>(c->wbuf);
+      HIP_TRY(mia::launch_typed_split(W0, type, reinterpret_cast<_Float16 *>(w),
+                                      reinterpret_cast<_Float16 *>(w + bw),
+                                      reinterpret_cast<float *>(w + 2 * bw), rows0, K, s));
+      p.w0 = reinterpret_cast<const uint8_t *>(w);
+    }
+    p.lo_bytes = bw;
+    p.row_scale = reinterpret_cast<const float *>(p.w0 + 2 * bw);
+  }
+  mia::gemm_plan(p, c->num_cus, plain_split);
   if (p.ksplit > 1) {
     if (int rc = ensure_gemm_work(c, (size_t)p.ksplit * S * p.N * sizeof(float))) return rc;
     p.part = reinterpret_cast<float *>(c->gemm_work);
   }
-  hipEvent_t ev0, ev1;
-  if (int rc = prof_pair(c, 3, &ev0, &ev1)) return rc;
-  HIP_TRY(mia::launch_q4_gemm(p, mode, c->num_cus, s, ev0, ev1));
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  if (type == MIA_TYPE_Q4_0) {
+    if (int rc = prof_pair(c, 3, &ev0, &ev1)) return rc;
+  }
+  HIP_TRY(mia::launch_gemm(p, mode, s, ev0, ev1));
+  return MIA_OK;
+}
+
+// Y [S][N] = X [S][K] . W^T for the K or V matrix of a layer (a type other than
+// Q4_0) from X's planes: [Xhi; Xlo] . Whi^T in one fp16 GEMM of 2S columns and,
+// for hi + lo weights, Xhi . Wlo^T in another, summed by the combine kernel.
+// The rings hold these sums rounded to fp16, so their rounding is kept as it
+// is: gemm_impl's sums are as close to the exact ones (3.0e-7 of a row against
+// 4.1e-7 here, 4096 values), but would move 0.3 % of the cached values to the
+// other fp16 neighbour.
+int kv_projection(DevCtx *c, int type, const void *W, const _Float16 *planes, int N, int K, int S,
+                  float *Y, hipStream_t s, bool packed) {
+  const bool lo = gemm_two_planes(type);
+  const size_t bp = packed ? 0 : typed_planes_bytes(type, N, K), bw = al256((size_t)N * K * 2);
+  const size_t bc = al256((size_t)2 * S * N * 4);
+  if (int rc = ensure_lt_buf(c, bp + (lo ? 2 : 1) * bc)) return rc;
+  if (int rc = ensure_lt(c)) return rc;
+  char *w = reinterpret_cast<char *>(c->lt_buf);
+  char *wp = packed ? reinterpret_cast<char *>(const_cast<void *>(W)) : w;
+  _Float16 *whi = reinterpret_cast<_Float16 *>(wp);
+  _Float16 *wlo = lo ? reinterpret_cast<_Float16 *>(wp + bw) : nullptr;
+  float *rs = lo ? reinterpret_cast<float *>(wp + 2 * bw) : nullptr;
+  float *C1 = reinterpret_cast<float *>(w + bp);
+  float *C2 = lo ? reinterpret_cast<float *>(w + bp + bc) : nullptr;
+  if (!packed) HIP_TRY(mia::launch_typed_split(W, type, whi, wlo, rs, N, K, s));
+  if (int rc = lt_gemm(c, N, 2 * S, K, whi, planes, C1, s)) return rc;
+  if (lo)
+    if (int rc = lt_gemm(c, N, S, K, wlo, planes, C2, s)) return rc;
+  HIP_TRY(mia::launch_hilo_combine(C1, C2, rs, Y, S, N, s));
   return MIA_OK;
 }
 
@@ -1116,8 +1204,8 @@ int mia_q4_0_gemm_f32(const void *W, const float *X, float *Y, int out_dim, int 
   if (int rc = check_align16(X, Y, nullptr, nullptr)) return rc;
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
-  return gemm_impl(c, W, nullptr, nullptr, out_dim, 0, 0, X, in_dim, S, Y, nullptr, nullptr,
-                   mia::kGemmStore, pick_stream(c, stream));
+  return gemm_impl(c, MIA_TYPE_Q4_0, W, nullptr, nullptr, out_dim, 0, 0, X, in_dim, S, Y, nullptr,
+                   nullptr, mia::kGemmStore, pick_stream(c, stream), false);
 }
 
 int mia_q4_0_pack_gemm(const void *W, void *Wp, int out_dim, int in_dim, void *stream) {
@@ -1145,12 +1233,93 @@ int mia_q4_0_gemm_packed_f32(const void *Wp, const float *X, float *Y, int out_d
   if (int rc = check_align16(X, Y, nullptr, nullptr)) return rc;
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
-  return gemm_impl(c, Wp, nullptr, nullptr, out_dim, 0, 0, X, in_dim, S, Y, nullptr, nullptr,
-                   mia::kGemmStore, pick_stream(c, stream), false, nullptr, nullptr, true);
+  return gemm_impl(c, MIA_TYPE_Q4_0, Wp, nullptr, nullptr, out_dim, 0, 0, X, in_dim, S, Y, nullptr,
+                   nullptr, mia::kGemmStore, pick_stream(c, stream), true);
 }
 
-// (every row count, dim, kv_dim and hidden, is a multiple of 64 here, as the
-// tile layout needs)
+// The prefill layer (mistral_ane_prefill.h:1081-1110) on checked arguments:
+// ws / types are wq, wk, wv, wo, w1, w2, w3.
+static int layer_run(DevCtx *c, float *X, const void *const (&ws)[7], const int (&types)[7],
+                     const float *rms_att, const float *rms_ffn, const float *theta_inv,
+                     uint16_t *k_layer, uint16_t *v_layer, int dim, int hidden, int n_kv_heads,
+                     float eps, int max_seq, int start_pos, int S, hipStream_t s, bool packed) {
+  const int kv_dim = n_kv_heads * kHD;
+  // gate and up in one launch, ending in the SwiGLU product
+  const bool fused_ffn = types[4] == types[6] && !gemm_two_planes(types[4]);
+  // Q [S][dim] | K, V [S][kv_dim] | A [S][dim] | H planes [2][S][hidden] fp16,
+  // or, without the fused launch, G and U [S][hidden]; the normalised rows
+  // (the QKV and W1 / W3 inputs) only exist as the GEMM's hi + lo planes in
+  // split_work, written there by the RMSNorm, and the SwiGLU output H (W2's
+  // input) only as the planes after A.
+  const size_t bd = al256((size_t)S * dim * 4), bk = al256((size_t)S * kv_dim * 4),
+               bh = al256((size_t)S * hidden * 4);
+  if (int rc = ensure_layer_work(c, 2 * bd + 2 * bk + (fused_ffn ? 1 : 2) * bh)) return rc;
+  if (int rc = ensure_split_work(c, (size_t)S * dim * 4)) return rc;  // [2][S][dim] fp16
+  char *w = reinterpret_cast<char *>(c->layer_work);
+  float *Q = reinterpret_cast<float *>(w);
+  float *K = reinterpret_cast<float *>(w + bd);
+  float *V = reinterpret_cast<float *>(w + bd + bk);
+  float *A = reinterpret_cast<float *>(w + bd + 2 * bk);
+  float *G = reinterpret_cast<float *>(w + 2 * bd + 2 * bk);
+  float *U = reinterpret_cast<float *>(w + 2 * bd + 2 * bk + bh);
+  _Float16 *const h_planes = reinterpret_cast<_Float16 *>(G);
+  _Float16 *const xn_hi = reinterpret_cast<_Float16 *>(c->split_work);
+  _Float16 *const xn_lo = xn_hi + (size_t)S * dim;
+  HIP_TRY(mia::launch_rmsnorm_split(xn_hi, xn_lo, X, rms_att, dim, S, eps, s));
+  // Q, K and V: one launch when all are Q4_0
+  const bool one_qkv =
+      types[0] == MIA_TYPE_Q4_0 && types[1] == MIA_TYPE_Q4_0 && types[2] == MIA_TYPE_Q4_0;
+  if (int rc = gemm_impl(c, types[0], ws[0], one_qkv ? ws[1] : nullptr, one_qkv ? ws[2] : nullptr,
+                         dim, one_qkv ? kv_dim : 0, one_qkv ? kv_dim : 0, nullptr, dim, S, Q,
+                         one_qkv ? K : nullptr, one_qkv ? V : nullptr, mia::kGemmStore, s, packed,
+                         /*reuse_split=*/true, nullptr, nullptr, /*plain_split=*/one_qkv))
+    return rc;
+  for (int i = 1; i < 3 && !one_qkv; ++i) {
+    float *const y = i == 1 ? K : V;
+    if (types[i] != MIA_TYPE_Q4_0) {
+      if (int rc = kv_projection(c, types[i], ws[i], xn_hi, kv_dim, dim, S, y, s, packed)) return rc;
+    } else if (int rc = gemm_impl(c, types[i], ws[i], nullptr, nullptr, kv_dim, 0, 0, nullptr, dim, S,
+                                  y, nullptr, nullptr, mia::kGemmStore, s, packed,
+                                  /*reuse_split=*/true, nullptr, nullptr, /*plain_split=*/true)) {
+      return rc;
+    }
+  }
+  // apply_rope_batch, kv_write_batch, attention_batch (:1097-1098): every
+  // token's K/V go into the ring first and each query attends the ring as
+  // it then stands; the (cos, sin) table of the positions lands in the work
+  // buffer, from which the attention kernel rotates Q.
+  if (int rc = ensure_work(c, (size_t)S * kHD * sizeof(float))) return rc;
+  float *cs = reinterpret_cast<float *>(c->work);
+  HIP_TRY(mia::launch_rope_to_ring(K, V, theta_inv, S, start_pos, n_kv_heads,
+                                   reinterpret_cast<_Float16 *>(k_layer),
+                                   reinterpret_cast<_Float16 *>(v_layer), max_seq, cs, s));
+  if (int rc = flash_impl(c, Q, cs, nullptr, nullptr, k_layer, v_layer, A, n_kv_heads, max_seq,
+                          start_pos, S, s))
+    return rc;
+  // X + A . Wo^T (vDSP_vadd after the GEMM: the sum rounded once more)
+  if (int rc = gemm_impl(c, types[3], ws[3], nullptr, nullptr, dim, 0, 0, A, dim, S, X, nullptr,
+                         nullptr, mia::kGemmAdd, s, packed))
+    return rc;
+  HIP_TRY(mia::launch_rmsnorm_split(xn_hi, xn_lo, X, rms_ffn, dim, S, eps, s));
+  if (fused_ffn) {
+    if (int rc = gemm_impl(c, types[4], ws[4], ws[6], nullptr, hidden, hidden, 0, nullptr, dim, S,
+                           nullptr, nullptr, nullptr, mia::kGemmSwiGlu, s, packed,
+                           /*reuse_split=*/true, nullptr, h_planes))
+      return rc;
+    return gemm_impl(c, types[5], ws[5], nullptr, nullptr, dim, 0, 0, nullptr, hidden, S, X,
+                     nullptr, nullptr, mia::kGemmAdd, s, packed, false, h_planes);
+  }
+  if (int rc = gemm_impl(c, types[4], ws[4], nullptr, nullptr, hidden, 0, 0, nullptr, dim, S, G,
+                         nullptr, nullptr, mia::kGemmStore, s, packed, /*reuse_split=*/true))
+    return rc;
+  if (int rc = gemm_impl(c, types[6], ws[6], nullptr, nullptr, hidden, 0, 0, nullptr, dim, S, U,
+                         nullptr, nullptr, mia::kGemmStore, s, packed, /*reuse_split=*/true))
+    return rc;
+  HIP_TRY(mia::launch_silu_mul(G, U, (long)S * hidden, s));
+  return gemm_impl(c, types[5], ws[5], nullptr, nullptr, dim, 0, 0, G, hidden, S, X, nullptr,
+                   nullptr, mia::kGemmAdd, s, packed);
+}
+
 static int prefill_layer_impl(float *X, const mia_layer_weights *lw, const float *theta_inv,
                        uint16_t *k_layer, uint16_t *v_layer, int dim, int hidden, int n_heads,
                        int n_kv_heads, float eps, int max_seq, int start_pos, int S, void *stream,
@@ -1174,57 +1343,11 @@ static int prefill_layer_impl(float *X, const mia_layer_weights *lw, const float
   if (int rc = check_align16(v_layer, nullptr, nullptr, nullptr)) return rc;
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
-  hipStream_t s = pick_stream(c, stream);
-  const int kv_dim = n_kv_heads * kHD;
-  // Q [S][dim] | K, V [S][kv_dim] | A [S][dim] | G [S][hidden] | H planes
-  // [2][S][hidden] fp16; the normalised rows (the QKV and W1 / W3 inputs) only
-  // exist as the GEMM's hi + lo planes in split_work, written there by the
-  // RMSNorm, and the SwiGLU output H (W2's input) only as the planes after G.
-  auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  const size_t bd = al((size_t)S * dim * 4), bk = al((size_t)S * kv_dim * 4),
-               bh = al((size_t)S * hidden * 4);
-  if (int rc = ensure_layer_work(c, 2 * bd + 2 * bk + 2 * bh)) return rc;
-  if (int rc = ensure_split_work(c, (size_t)S * dim * 4)) return rc;  // [2][S][dim] fp16
-  char *w = reinterpret_cast<char *>(c->layer_work);
-  float *Q = reinterpret_cast<float *>(w);
-  float *K = reinterpret_cast<float *>(w + bd);
-  float *V = reinterpret_cast<float *>(w + bd + bk);
-  float *A = reinterpret_cast<float *>(w + bd + 2 * bk);
-  float *G = reinterpret_cast<float *>(w + 2 * bd + 2 * bk);
-  _Float16 *const h_planes = reinterpret_cast<_Float16 *>(w + 2 * bd + 2 * bk + bh);
-  _Float16 *const xn_hi = reinterpret_cast<_Float16 *>(c->split_work);
-  _Float16 *const xn_lo = xn_hi + (size_t)S * dim;
-  // mistral_ane_prefill.h:1092-1110
-  HIP_TRY(mia::launch_rmsnorm_split(xn_hi, xn_lo, X, lw->rms_att, dim, S, eps, s));
-  if (int rc = gemm_impl(c, lw->wq, lw->wk, lw->wv, dim, kv_dim, kv_dim, nullptr, dim, S, Q, K,
-                         V, mia::kGemmStore, s, /*reuse_split=*/true, nullptr, nullptr, packed))
-    return rc;
-  // apply_rope_batch, kv_write_batch, attention_batch (:1097-1098): every
-  // token's K/V go into the ring first and each query attends the ring as
-  // it then stands; the (cos, sin) table of the positions lands in the work
-  // buffer, from which the attention kernel rotates Q.
-  if (int rc = ensure_work(c, (size_t)S * kHD * sizeof(float))) return rc;
-  float *cs = reinterpret_cast<float *>(c->work);
-  HIP_TRY(mia::launch_rope_to_ring(K, V, theta_inv, S, start_pos, n_kv_heads,
-                                   reinterpret_cast<_Float16 *>(k_layer),
-                                   reinterpret_cast<_Float16 *>(v_layer), max_seq, cs, s));
-  if (int rc = flash_impl(c, Q, cs, nullptr, nullptr, k_layer, v_layer, A, n_kv_heads, max_seq,
-                          start_pos, S, s))
-    return rc;
-  if (int rc = gemm_impl(c, lw->wo, nullptr, nullptr, dim, 0, 0, A, dim, S, X, nullptr, nullptr,
-                         mia::kGemmAdd, s, false, nullptr, nullptr, packed))
-    return rc;
-  HIP_TRY(mia::launch_rmsnorm_split(xn_hi, xn_lo, X, lw->rms_ffn, dim, S, eps, s));
-  if (int rc = gemm_impl(c, lw->w1, nullptr, nullptr, hidden, 0, 0, nullptr, dim, S, G, nullptr,
-                         nullptr, mia::kGemmStore, s, /*reuse_split=*/true, nullptr, nullptr,
-                         packed))
-    return rc;
-  if (int rc = gemm_impl(c, lw->w3, nullptr, nullptr, hidden, 0, 0, nullptr, dim, S, G, nullptr,
-                         nullptr, mia::kGemmSiluMul, s, /*reuse_split=*/true, nullptr, h_planes,
-                         packed))
-    return rc;
-  return gemm_impl(c, lw->w2, nullptr, nullptr, dim, 0, 0, nullptr, hidden, S, X, nullptr,
-                   nullptr, mia::kGemmAdd, s, false, h_planes, nullptr, packed);
+  const void *const ws[7] = {lw->wq, lw->wk, lw->wv, lw->wo, lw->w1, lw->w2, lw->w3};
+  const int types[7] = {MIA_TYPE_Q4_0, MIA_TYPE_Q4_0, MIA_TYPE_Q4_0, MIA_TYPE_Q4_0,
+                        MIA_TYPE_Q4_0, MIA_TYPE_Q4_0, MIA_TYPE_Q4_0};
+  return layer_run(c, X, ws, types, lw->rms_att, lw->rms_ffn, theta_inv, k_layer, v_layer, dim,
+                   hidden, n_kv_heads, eps, max_seq, start_pos, S, pick_stream(c, stream), packed);
 }
 
 int mia_prefill_layer(float *X, const mia_layer_weights *lw, const float *theta_inv,
@@ -1254,59 +1377,6 @@ static int check_typed(int type, int in_dim, const void *W) {
   const uintptr_t need = (type == MIA_TYPE_Q4_0 || type == MIA_TYPE_Q6_K) ? 2 : 16;
   if ((uintptr_t)W & (need - 1))
     return set_err(MIA_ERR_INVALID, "W of type %d must be %d-byte aligned", type, (int)need);
-  return MIA_OK;
-}
-
-// Y [S][N] (+)= X [S][K] . W^T for a weight type other than Q4_0, on fp16
-// MFMA with fp32 accumulation (rocBLAS gemm_ex): X as fp16 hi + lo planes
-// (launch_split_hilo), W as its fp16 values (Q4_K, F16: exact) or as row-scaled
-// hi + lo planes (Q6_K, F32: launch_typed_split).  C1 = [Xhi; Xlo] . Whi^T in
-// one GEMM of 2S columns, C2 = Xhi . Wlo^T; the combine kernel sums the parts
-// (the Xlo . Wlo term, ~2^-22 of the product, is dropped).  rocBLAS is
-// column-major: C^T [N][cols] = (W^T [K][N])^T . B^T [K][cols], so W is the
-// transposed A operand with lda K and C's leading dimension is N.
-static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
-
-// The typed GEMM's packed form of a matrix of a type other than Q4_0: the fp16
-// hi plane [N][K], then for Q6_K / F32 the lo plane [N][K] and the row scales
-// [N] fp32, each at a 256-byte aligned offset (launch_typed_split's output).
-static size_t typed_planes_bytes(int type, int N, int K) {
-  const bool lo = !mia::typed_is_f16_exact(type);
-  const size_t bw = al256((size_t)N * K * 2);
-  return lo ? 2 * bw + al256((size_t)N * 4) : bw;
-}
-
-// reuse_x: split_work already holds X's planes (the call before split the
-// same X on this stream), and X is not read.  packed: W is in the packed form
-// (Q4_0: mia_q4_0_pack_gemm's tile layout; other types: the planes above).
-static int typed_gemm_impl(DevCtx *c, const void *W, int type, const float *X, float *Y, int N,
-                           int K, int S, bool add, hipStream_t s, bool reuse_x = false,
-                           bool packed = false) {
-  if (type == MIA_TYPE_Q4_0)
-    return gemm_impl(c, W, nullptr, nullptr, N, 0, 0, X, K, S, Y, nullptr, nullptr,
-                     add ? mia::kGemmAdd : mia::kGemmStore, s, reuse_x, nullptr, nullptr, packed);
-  const bool lo = !mia::typed_is_f16_exact(type);
-  const size_t bp = packed ? 0 : typed_planes_bytes(type, N, K);
-  const size_t bc1 = al256((size_t)2 * S * N * 4), bc2 = al256((size_t)S * N * 4);
-  if (int rc = ensure_wbuf(c, bp + bc1 + (lo ? bc2 : 0))) return rc;
-  if (int rc = ensure_split_work(c, (size_t)2 * S * K * sizeof(_Float16))) return rc;
-  if (int rc = ensure_lt(c)) return rc;
-  char *w = reinterpret_cast<char *>(c->wbuf);
-  char *planes = packed ? reinterpret_cast<char *>(const_cast<void *>(W)) : w;
-  const size_t bw = al256((size_t)N * K * 2);
-  _Float16 *whi = reinterpret_cast<_Float16 *>(planes);
-  _Float16 *wlo = lo ? reinterpret_cast<_Float16 *>(planes + bw) : nullptr;
-  float *rs = lo ? reinterpret_cast<float *>(planes + 2 * bw) : nullptr;
-  float *C1 = reinterpret_cast<float *>(w + bp);
-  float *C2 = lo ? reinterpret_cast<float *>(w + bp + bc1) : nullptr;
-  _Float16 *xhi = reinterpret_cast<_Float16 *>(c->split_work);  // [2][S][K]: hi, then lo
-  if (!packed) HIP_TRY(mia::launch_typed_split(W, type, whi, wlo, rs, N, K, s));
-  if (!reuse_x)
-    HIP_TRY(mia::launch_split_hilo(X, (long)S * K, xhi, xhi + (size_t)S * K, c->num_cus, s));
-  if (int rc = lt_gemm(c, N, 2 * S, K, whi, xhi, C1, s)) return rc;
-  if (lo)
-    if (int rc = lt_gemm(c, N, S, K, wlo, xhi, C2, s)) return rc;
-  HIP_TRY(mia::launch_hilo_combine(C1, C2, rs, Y, S, N, add, s));
   return MIA_OK;
 }
 
@@ -1364,7 +1434,8 @@ int mia_gemm_f32(const void *W, int type, const float *X, float *Y, int out_dim,
   if (int rc = check_align16(X, Y, nullptr, nullptr)) return rc;
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
-  return typed_gemm_impl(c, W, type, X, Y, out_dim, in_dim, S, false, pick_stream(c, stream));
+  return gemm_impl(c, type, W, nullptr, nullptr, out_dim, 0, 0, X, in_dim, S, Y, nullptr, nullptr,
+                   mia::kGemmStore, pick_stream(c, stream), false);
 }
 
 static int typed_layer_impl(float *X, const mia_layer_weights_typed *lw, const float *theta_inv,
@@ -1412,48 +1483,8 @@ static int typed_layer_impl(float *X, const mia_layer_weights_typed *lw, const f
   if (int rc = check_align16(v_layer, nullptr, nullptr, nullptr)) return rc;
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
-  hipStream_t s = pick_stream(c, stream);
-  // XN, Q, A [S][dim] | K, V [S][kv_dim] | G, U [S][hidden], all fp32
-  auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  const size_t bd = al((size_t)S * dim * 4), bk = al((size_t)S * kv_dim * 4),
-               bh = al((size_t)S * hidden * 4);
-  if (int rc = ensure_layer_work(c, 3 * bd + 2 * bk + 2 * bh)) return rc;
-  char *w = reinterpret_cast<char *>(c->layer_work);
-  float *XN = reinterpret_cast<float *>(w);
-  float *Q = reinterpret_cast<float *>(w + bd);
-  float *A = reinterpret_cast<float *>(w + 2 * bd);
-  float *K = reinterpret_cast<float *>(w + 3 * bd);
-  float *V = reinterpret_cast<float *>(w + 3 * bd + bk);
-  float *G = reinterpret_cast<float *>(w + 3 * bd + 2 * bk);
-  float *U = reinterpret_cast<float *>(w + 3 * bd + 2 * bk + bh);
-  // mistral_ane_prefill.h:1092-1110
-  HIP_TRY(mia::launch_rmsnorm(XN, X, lw->rms_att, dim, S, eps, s));
-  // (the normalised rows are split into fp16 planes once for Q, K and V)
-  if (int rc = typed_gemm_impl(c, lw->wq, lw->wq_type, XN, Q, dim, dim, S, false, s, false, packed))
-    return rc;
-  if (int rc = typed_gemm_impl(c, lw->wk, lw->wk_type, XN, K, kv_dim, dim, S, false, s, true, packed))
-    return rc;
-  if (int rc = typed_gemm_impl(c, lw->wv, lw->wv_type, XN, V, kv_dim, dim, S, false, s, true, packed))
-    return rc;
-  // apply_rope_batch, kv_write_batch, attention_batch, as mia_prefill_layer
-  if (int rc = ensure_work(c, (size_t)S * kHD * sizeof(float))) return rc;
-  float *cs = reinterpret_cast<float *>(c->work);
-  HIP_TRY(mia::launch_rope_to_ring(K, V, theta_inv, S, start_pos, n_kv_heads,
-                                   reinterpret_cast<_Float16 *>(k_layer),
-                                   reinterpret_cast<_Float16 *>(v_layer), max_seq, cs, s));
-  if (int rc = flash_impl(c, Q, cs, nullptr, nullptr, k_layer, v_layer, A, n_kv_heads, max_seq,
-                          start_pos, S, s))
-    return rc;
-  // X + A . Wo^T (vDSP_vadd after the GEMM: the sum rounded once more)
-  if (int rc = typed_gemm_impl(c, lw->wo, lw->wo_type, A, X, dim, dim, S, true, s, false, packed))
-    return rc;
-  HIP_TRY(mia::launch_rmsnorm(XN, X, lw->rms_ffn, dim, S, eps, s));
-  if (int rc = typed_gemm_impl(c, lw->w1, lw->w1_type, XN, G, hidden, dim, S, false, s, false, packed))
-    return rc;
-  if (int rc = typed_gemm_impl(c, lw->w3, lw->w3_type, XN, U, hidden, dim, S, false, s, true, packed))
-    return rc;
-  HIP_TRY(mia::launch_silu_mul(G, U, (long)S * hidden, s));
-  return typed_gemm_impl(c, lw->w2, lw->w2_type, G, X, dim, hidden, S, true, s, false, packed);
+  return layer_run(c, X, ws, types, lw->rms_att, lw->rms_ffn, theta_inv, k_layer, v_layer, dim,
+                   hidden, n_kv_heads, eps, max_seq, start_pos, S, pick_stream(c, stream), packed);
 }
 
 int mia_prefill_layer_typed(float *X, const mia_layer_weights_typed *lw, const float *theta_inv,
@@ -1516,8 +1547,8 @@ int mia_gemm_packed_f32(const void *Wp, int type, const float *X, float *Y, int 
   if (int rc = check_align16(X, Y, nullptr, nullptr)) return rc;
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
-  return typed_gemm_impl(c, Wp, type, X, Y, out_dim, in_dim, S, false, pick_stream(c, stream),
-                         false, true);
+  return gemm_impl(c, type, Wp, nullptr, nullptr, out_dim, 0, 0, X, in_dim, S, Y, nullptr, nullptr,
+                   mia::kGemmStore, pick_stream(c, stream), true);
 }
 
 int mia_quantize_q8_0(const float *x, void *out_q8, int n, void *stream) {

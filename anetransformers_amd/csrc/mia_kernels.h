@@ -158,9 +158,23 @@ hipError_t launch_scale_rows(_Float16 *base, long n_rows, int row_elems, int eve
                              float factor, hipStream_t s);
 
 // Prefill layer pieces (mia_prefill.hip).  Y[S][N] = A[S][K] . W^T with W up
-// to three Q4_0 matrices stacked as virtual rows (as Q4MatvecParams); K a
-// multiple of 64; A 16-byte aligned with lda a multiple of 4.
-enum { kGemmStore = 0, kGemmAdd = 1, kGemmSiluMul = 2 };
+// to three matrices of one type stacked as virtual rows (as Q4MatvecParams).
+enum { kGemmStore = 0, kGemmAdd = 1, kGemmSwiGlu = 2 };
+// Where the weights come from: Q4_0 in the GEMM tile layout of launch_q4_pack,
+// Q4_0 or Q4_K as GGUF stores them, fp16 values [N][K], or, one matrix per
+// launch and not kGemmSwiGlu, fp16 hi + lo planes with row scales
+// (launch_typed_split) or Q6_K regrouped (launch_q6k_regroup).
+enum {
+  kGemmQ40Tile = 0,
+  kGemmQ40 = 1,
+  kGemmQ4K = 2,
+  kGemmF16 = 3,
+  kGemmF16x2 = 4,
+  kGemmQ6K = 5
+};
+// The K split of a launch falls on multiples of this many K values, whatever
+// the source (K a multiple of 32; of 64 for Q4_0, of 256 for Q4_K).
+__host__ __device__ constexpr int gemm_k_unit(int K) { return K % 64 == 0 ? 64 : 32; }
 struct GemmParams {
   // the fp32 activations as fp16 hi + lo planes, [S][K] each (launch_split_hilo)
   const _Float16 *ahi, *alo;
@@ -168,29 +182,29 @@ struct GemmParams {
   int rows0, rows01, N;  // rows of w0, of w0 + w1, and in all
   int K, S;
   // kGemmStore: y0 [S][rows0], y1 [S][rows01 - rows0], y2 [S][N - rows01];
-  // kGemmAdd: y0 [S][N] += result; kGemmSiluMul: y0 [S][N] holds the gate and
-  // becomes gate * sigmoid(gate) * result.
+  // kGemmAdd: y0 [S][N] += result; kGemmSwiGlu: w0 (gate) and w1 (up) of rows0
+  // rows each, and gate * sigmoid(gate) * up goes out as fp16 hi + lo planes
+  // [S][rows0] (the next GEMM's input, launch_split_hilo's split).
   float *y0, *y1, *y2;
-  // K split over blockIdx.z (1: none).  With ksplit > 1 the partial products
-  // go to part [ksplit][S][N] and a second kernel sums them in split order
-  // and applies the epilogue.
-  int ksplit;
-  float *part;
-  // kGemmSiluMul only: when set, the result goes out as fp16 hi + lo planes
-  // [S][N] (the next GEMM's input, launch_split_hilo's split) instead of
-  // into y0.
   _Float16 *ohi, *olo;
-  // w0, w1, w2 in the GEMM tile layout of launch_q4_pack (row counts and K
-  // multiples of 64) instead of the GGUF layout
-  int packed;
+  int src;  // kGemmQ40Tile .. kGemmQ6K (tiles: row counts and K multiples of 64)
+  size_t lo_bytes;          // kGemmF16x2: from the hi to the lo plane
+  const float *row_scale;   // kGemmF16x2, kGemmQ6K: [N]
+  // gemm_plan's choice: 32 tm tokens per workgroup, K split in ksplit.  With
+  // ksplit > 1 the partial products go to part [ksplit][S][N] and a second
+  // kernel sums them in split order and applies the epilogue.
+  int tm, ksplit;
+  float *part;
 };
-long gemm_tiles(int N, int S);
 // Q4_0 [N][K / 32] in the GGUF layout -> the GEMM tile layout (same size;
 // N and K multiples of 64, src 4-byte and dst 16-byte aligned, no overlap).
 hipError_t launch_q4_pack(const void *src, void *dst, int N, int K, hipStream_t s);
-int gemm_pick_ksplit(int N, int K, int S, int num_cus);
-hipError_t launch_q4_gemm(const GemmParams &p, int mode, int num_cus, hipStream_t s,
-                          hipEvent_t ev0, hipEvent_t ev1);
+// Sets tm and ksplit from N, K, S and the kind of weights.  plain: the K split
+// from N, K and S alone, by a fixed rule (sums that are rounded to fp16 and
+// kept, like a ring's keys and values, then do not move with the tuning).
+void gemm_plan(GemmParams &p, int num_cus, bool plain);
+hipError_t launch_gemm(const GemmParams &p, int mode, hipStream_t s, hipEvent_t ev0,
+                       hipEvent_t ev1);
 // x [n] fp32 -> hi, lo [n] fp16 with x = hi + lo to ~2^-22 (n a multiple of 8).
 hipError_t launch_split_hilo(const float *x, long n, _Float16 *hi, _Float16 *lo, int num_cus,
                              hipStream_t s);
@@ -217,10 +231,18 @@ hipError_t launch_typed_dequant(const void *W, int type, float *out, int rows, i
 bool typed_is_f16_exact(int type);
 hipError_t launch_typed_split(const void *W, int type, _Float16 *hi, _Float16 *lo, float *rscale,
                               int rows, int cols, hipStream_t s);
-// Y [S][N] (+)= rscale[n] * ((C1[s][n] + C1[S + s][n]) + C2[s][n]); C2 and
-// rscale null: Y (+)= C1[s][n] + C1[S + s][n].
+// Y [S][N] = rscale[n] * ((C1[s][n] + C1[S + s][n]) + C2[s][n]); C2 and
+// rscale null: Y = C1[s][n] + C1[S + s][n].
 hipError_t launch_hilo_combine(const float *C1, const float *C2, const float *rscale, float *Y,
-                               int S, int N, bool add, hipStream_t s);
+                               int S, int N, hipStream_t s);
+// Q6_K rows -> the GEMM's aligned form, rows x cols bytes (16-byte aligned), and
+// rscale [rows] as launch_typed_split gives it.  Per row and 64 values: 32
+// bytes of low nibbles (byte i: values i and 32 + i), then for each half h
+// (values 16 h .. and 32 + 16 h ..) the top bit pairs of the 16 values of
+// either block (two dwords: value 2 p at bits 2 p, value 2 p + 1 at bits
+// 16 + 2 p) and the two blocks' scales (fp32, d * scale / rscale).
+hipError_t launch_q6k_regroup(const void *W, uint8_t *out, float *rscale, int rows, int cols,
+                              hipStream_t s);
 // The decode layer's residual steps (mia_layer.hip): x += y, then out =
 // rmsnorm(x) (dim a multiple of 4, pointers 16-byte aligned); x += y.
 hipError_t launch_residual_rmsnorm(float *x, const float *y, const float *w, float *out, int dim,

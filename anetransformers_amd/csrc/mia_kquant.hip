@@ -21,10 +21,10 @@
 //   typed_matvec_kernel   the same for F16, F32 and Q4_0 with fp32 x, one
 //                         wave per row
 //   typed_dequant_kernel  the fp32 weight rows (dequant_weight_to_fp32_buf)
-//   typed_split_kernel    the prefill GEMM's fp16 operands: the fp16 values of
-//                         Q4_K / F16 weights, row-scaled hi + lo halves of
-//                         Q6_K / F32 weights, for rocBLAS gemm_ex
-//   hilo_combine_kernel   the GEMM's partial products summed (+ residual)
+//   typed_split_kernel    the prefill GEMM's fp16 planes (mia_gemm.hip): the
+//                         fp16 values of Q4_K / F16 weights, row-scaled hi +
+//                         lo halves of Q6_K / F32 weights
+//   hilo_combine_kernel   the K and V projections' partial products summed
 //   silu_mul_kernel       the SwiGLU product between the FFN GEMMs
 // Every matvec row sums its fp32 products in another order than the
 // reference's sgemv / four-lane NEON sums.  The matvecs are memory-bound:
@@ -775,6 +775,13 @@ __global__ void __launch_bounds__(256) typed_f16_kernel(const uint8_t *W, long r
   }
 }
 
+// 2^e scales a row whose largest |w| is m into [2^13, 2^14).
+__device__ __forceinline__ int row_exponent(float m) {
+  int ex = 0;
+  if (m > 0.f && m <= 3.4e38f) (void)frexpf(m, &ex);
+  return min(max(14 - ex, -60), 60);
+}
+
 template <int TYPE, bool LO>
 __global__ void __launch_bounds__(256) typed_split_kernel(const uint8_t *W, long row_bytes,
                                                           _Float16 *hi, _Float16 *lo,
@@ -797,9 +804,7 @@ __global__ void __launch_bounds__(256) typed_split_kernel(const uint8_t *W, long
       __syncthreads();
       m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
       __syncthreads();  // wmax is rewritten for the next row
-      int ex = 0;
-      if (m > 0.f && m <= 3.4e38f) (void)frexpf(m, &ex);
-      const int e = min(max(14 - ex, -60), 60);
+      const int e = row_exponent(m);
       scale = ldexpf(1.0f, e);
       if (threadIdx.x == 0) rscale[r] = ldexpf(1.0f, -e);
     }
@@ -826,12 +831,12 @@ __global__ void __launch_bounds__(256) typed_split_kernel(const uint8_t *W, long
   }
 }
 
-// Y [S][N] (+)= rscale[n] * ((C1 [S][N] + C1 [S + s][N]) + C2 [S][N]): the
+// Y [S][N] = rscale[n] * ((C1 [S][N] + C1 [S + s][N]) + C2 [S][N]): the
 // hi-activation and lo-activation products of the hi weights, plus the lo
 // weights' product (C2, rscale: null for fp16-valued weights).
 __global__ void __launch_bounds__(256) hilo_combine_kernel(const float *C1, const float *C2,
                                                            const float *rscale, float *Y, int S,
-                                                           int N, bool add) {
+                                                           int N) {
 #pragma clang fp contract(off)
   const long total = (long)S * N;
   if ((N & 3) == 0) {  // four outputs per thread (16-byte aligned rows)
@@ -840,15 +845,104 @@ __global__ void __launch_bounds__(256) hilo_combine_kernel(const float *C1, cons
       f4 v = reinterpret_cast<const f4 *>(C1)[i] + reinterpret_cast<const f4 *>(C1 + total)[i];
       if (C2) v = (v + reinterpret_cast<const f4 *>(C2)[i]) *
                   reinterpret_cast<const f4 *>(rscale)[(4 * i) % N >> 2];
-      f4 *y = reinterpret_cast<f4 *>(Y) + i;
-      *y = add ? *y + v : v;
+      reinterpret_cast<f4 *>(Y)[i] = v;
     }
     return;
   }
   for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long)gridDim.x * 256) {
     float v = C1[i] + C1[total + i];
     if (C2) v = (v + C2[i]) * rscale[i % N];
-    Y[i] = add ? Y[i] + v : v;
+    Y[i] = v;
+  }
+}
+
+// Q6_K -> the GEMM's aligned form (launch_q6k_regroup), one workgroup per row.
+// Reading a matrix and writing it as bytes instead of as hi + lo planes (210 /
+// 256 + 1 bytes a weight against 210 / 256 + 4) is what it saves.
+__global__ void __launch_bounds__(256) q6k_regroup_kernel(const uint8_t *W, long row_bytes,
+                                                          uint8_t *out, float *rscale, int cols) {
+  __shared__ float wmax[4];
+  const int r = blockIdx.x;
+  const uint8_t *wr = W + (size_t)r * row_bytes;
+  const int nchunk = cols >> 6;
+  // group 2 c + b of the row: block b of chunk c; 32 values, two scales
+  auto group = [&](int g, unsigned (&q)[8], float (&ds)[2]) {
+    Q6KRaw raw;
+    kq_load(wr, g, raw);
+    const int n0 = 32 * (g & 7), rr = n0 >> 6;
+    const int lo_sh = n0 < 128 ? 0 : 4, hi_sh = rr == 0 ? 0 : (rr == 1 ? 4 : (rr == 2 ? 2 : 6));
+    const u4 ql[2] = {raw.ql0, raw.ql1}, qh[2] = {raw.qh0, raw.qh1};
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      q[i] = ((ql[i >> 2][i & 3] >> lo_sh) & 0x0F0F0F0Fu) |
+             (((qh[i >> 2][i & 3] >> hi_sh) & 0x03030303u) << 4);
+    const float d = half_bits(raw.dh);
+    ds[0] = d * (float)(int)(signed char)(raw.sc2 & 0xFF);
+    ds[1] = d * (float)(int)(signed char)(raw.sc2 >> 8);
+  };
+  // the largest |w| = |ds| |q - 32| of a group
+  auto group_max = [&](const unsigned (&q)[8], const float (&ds)[2], float m) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      int lo = 63, hi = 0;
+#pragma unroll
+      for (int i = 4 * h; i < 4 * h + 4; ++i)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int v = (q[i] >> (8 * b)) & 0xFF;
+          lo = min(lo, v);
+          hi = max(hi, v);
+        }
+      m = fmaxf(m, fabsf(ds[h] * (float)max(hi - 32, 32 - lo)));
+    }
+    return m;
+  };
+  // chunk c's groups stay in registers from the maximum to the output, for as
+  // many chunks as there are threads; the rest of a longer row is read again
+  unsigned q[2][8];
+  float ds[2][2];
+  float m = 0.f;
+  const int own = threadIdx.x;  // this thread's chunks: own, own + 256, ...; own comes last here
+  for (int k = own < nchunk ? (nchunk - 1 - own) / 256 : -1; k >= 0; --k) {
+    const int c = own + 256 * k;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      group(2 * c + b, q[b], ds[b]);
+      m = group_max(q[b], ds[b], m);
+    }
+  }
+  m = wave_max(m);
+  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+  const int e = row_exponent(m);
+  const float scale = ldexpf(1.0f, e);
+  if (threadIdx.x == 0) rscale[r] = ldexpf(1.0f, -e);
+  for (int c = own; c < nchunk; c += 256) {
+    if (c != own) {
+      group(2 * c, q[0], ds[0]);
+      group(2 * c + 1, q[1], ds[1]);
+    }
+    unsigned low[8];
+    u4 *dst = reinterpret_cast<u4 *>(out + ((size_t)r * nchunk + c) * 64);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) low[i] = (q[0][i] & 0x0F0F0F0Fu) | (q[1][i] & 0x0F0F0F0Fu) << 4;
+    dst[0] = (u4){low[0], low[1], low[2], low[3]};
+    dst[1] = (u4){low[4], low[5], low[6], low[7]};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      unsigned top[2] = {0u, 0u}, sb[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {  // values 2 p, 2 p + 1 of the half's 16
+          const unsigned w = q[b][4 * h + (p >> 1)] >> (16 * (p & 1));
+          top[b] |= ((w >> 4) & 3u) << (2 * p) | ((w >> 12) & 3u) << (16 + 2 * p);
+        }
+        sb[b] = __builtin_bit_cast(unsigned, ds[b][h] * scale);
+      }
+      dst[2 + h] = (u4){top[0], top[1], sb[0], sb[1]};
+    }
   }
 }
 
@@ -1042,12 +1136,21 @@ hipError_t launch_typed_split(const void *W, int type, _Float16 *hi, _Float16 *l
 }
 
 hipError_t launch_hilo_combine(const float *C1, const float *C2, const float *rscale, float *Y,
-                               int S, int N, bool add, hipStream_t s) {
+                               int S, int N, hipStream_t s) {
   const long total = (long)S * N;
   long blocks = (total + 255) / 256;
   if (blocks > 8192) blocks = 8192;
   hipLaunchKernelGGL(hilo_combine_kernel, dim3((unsigned)blocks), dim3(256), 0, s, C1, C2, rscale,
-                     Y, S, N, add);
+                     Y, S, N);
+  return hipGetLastError();
+}
+
+hipError_t launch_q6k_regroup(const void *W, uint8_t *out, float *rscale, int rows, int cols,
+                              hipStream_t s) {
+  const long rb = typed_row_bytes(kTypeQ6K, cols);
+  if (rb == 0 || rows <= 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(q6k_regroup_kernel, dim3(rows), dim3(256), 0, s,
+                     reinterpret_cast<const uint8_t *>(W), rb, out, rscale, cols);
   return hipGetLastError();
 }
 

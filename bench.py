@@ -892,8 +892,9 @@ def typed_leg(lib, steps: int, warmup: int) -> dict:
             "workload": "mia_prefill_layer_typed_packed x 32, S 512 after 1536 cached: the "
                         "weights in the GEMM operand form made once at set-up (mia_gemm_pack: "
                         "fp16 values of Q4_K, row-scaled hi + lo halves of Q6_K, 18 GB), fp16 "
-                        "MFMA GEMMs (hipBLASLt, each shape's algorithm picked by timing on its first "
-                        "call, in the warm-up) on the activations' hi + lo halves",
+                        "MFMA GEMMs on the activations' hi + lo halves (K and V projections: "
+                        "hipBLASLt, each shape's algorithm picked by timing on its first call, in "
+                        "the warm-up)",
             "value": round(N_LAYERS * layer_flop / (pf_ms * 1e-3) / 1e12, 3), "unit": "TFLOP/s",
             "ms_per_step": round(pf_ms, 3), "flop_per_layer": layer_flop,
             "per_call_conversion_ms_per_step": round(pf_conv_ms, 3),
@@ -1259,7 +1260,7 @@ def main() -> int:
         pl_steps = max(args.steps // 4, 2)
         pl_ms = timed(lib, pl.step, pl_steps, 1)
         g_n, g_ms = kernel_stats(lib, pl.step, pl_steps, 3)
-        gemm_tfs = (LAYER_GEMM_FLOP / 5) / (g_ms * 1e-3) / 1e12
+        gemm_tfs = LAYER_GEMM_FLOP * N_LAYERS * pl_steps / (g_n * g_ms * 1e-3) / 1e12
         layer_flop = LAYER_GEMM_FLOP + PF_FLOP_PER_LAYER
         log(f"prefill layer: {pl_ms:.2f} ms/step ({N_LAYERS * layer_flop / (pl_ms * 1e-3) / 1e12:.1f} "
             f"TFLOP/s), GEMM kernel {g_ms * 1e3:.1f} us avg ({gemm_tfs:.1f} TFLOP/s)")

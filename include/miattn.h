@@ -363,26 +363,21 @@ int mia_matvec_q8(const void *W, int type, const void *x_q8, float *y, int out_d
 /* tiled_q4_gemm for every type (mistral/mistral_ane_prefill.h:1018-1042):
  * Y[S][out_dim] = X[S][in_dim] . W^T, fp32 X and Y (dev, 16-byte aligned).
  * Q4_0 is mia_q4_0_gemm_f32.  The other types multiply on fp16 MFMA with fp32
- * accumulation (hipBLASLt; the algorithm of each GEMM shape is timed and
- * picked on the shape's first call in the process, which therefore waits for
- * the stream once; later calls of the shape reuse it, so repeated calls give
- * bit-identical results), within fp32 rounding of the reference's
- * dequantise + cblas_sgemm: X is split into fp16 hi + lo halves, as for Q4_0;
- * Q4_K and F16 weights are fp16 values and enter exactly; Q6_K and F32
- * weights are scaled per row by a power of two and split into hi + lo halves
- * (2^-22 relative).  Per-device work areas: out_dim * in_dim * 2 bytes
- * (twice that for Q6_K / F32), 12 * S * out_dim bytes and a 64 MiB GEMM
- * workspace.  Range as
- * mia_q4_0_gemm_f32's: every |x| below 65504, below 2^-3 carried to 2^-25
- * absolute. */
+ * accumulation, within fp32 rounding of the reference's dequantise +
+ * cblas_sgemm: X is split into fp16 hi + lo halves, as for Q4_0; Q4_K and F16
+ * weights are fp16 values and enter exactly; Q6_K and F32 weights are scaled
+ * per row by a power of two and split into hi + lo halves (2^-22 relative).
+ * Repeated calls give bit-identical results.  Per-device work areas: Q6_K
+ * out_dim * in_dim bytes, F32 four times that, and up to 64 * S * out_dim
+ * bytes of partial products when K is split.  Range as mia_q4_0_gemm_f32's:
+ * every |x| below 65504, below 2^-3 carried to 2^-25 absolute. */
 int mia_gemm_f32(const void *W, int type, const float *X, float *Y, int out_dim, int in_dim,
                  int S, void *stream);
 
 /* The same weights converted once, at load time, into the GEMM's operand form
  * (no reference counterpart; the reference dequantises per call,
  * mistral/mistral_ane_prefill.h:1018-1042), so that the per-call conversion
- * drops out: results are bit-identical to mia_gemm_f32's in the same process
- * (the same GEMM algorithm for the shape).  Q4_0 is
+ * drops out: results are bit-identical to mia_gemm_f32's.  Q4_0 is
  * mia_q4_0_pack_gemm's tile layout (out_dim and in_dim multiples of 64, the
  * size of the GGUF form); Q4_K and F16 become their fp16 values [out_dim]
  * [in_dim] (4x / 1x the Q4_K / F16 bytes); Q6_K and F32 the row-scaled fp16
@@ -406,11 +401,16 @@ typedef struct {
 /* blas_prefill_layer (mistral/mistral_ane_prefill.h:1081-1110) with each
  * matrix of its own type, as mia_prefill_layer otherwise (same arguments,
  * attention step and ring semantics).  A layer whose seven matrices are all
- * Q4_0 is mia_prefill_layer; any other mix multiplies each matrix as
- * mia_gemm_f32 does for its type, with the activations in fp32 and the
- * SwiGLU product
- * gate * (1 / (1 + exp(-gate))) * up (silu_mul_neon, mistral_model.h:
- * 174-199) in between. */
+ * Q4_0 is mia_prefill_layer; any other mix multiplies Wq, Wo, W1, W2 and W3
+ * (and Wk, Wv where they are Q4_0) as mia_gemm_f32 does for their types, with
+ * the activations in fp32 and the SwiGLU product gate * (1 / (1 +
+ * exp(-gate))) * up (silu_mul_neon, mistral_model.h:174-199) in between.  Wk
+ * and Wv of other types multiply the same fp16 planes through hipBLASLt: the
+ * algorithm of each shape is timed and picked on the shape's first call in
+ * the process, which therefore waits for the stream once; later calls of the
+ * shape reuse it and repeat their results bit for bit.  Work areas of these
+ * two: n_kv_heads * 128 * dim * 2 bytes (twice that for Q6_K / F32),
+ * 12 * S * n_kv_heads * 128 bytes and a 64 MiB workspace. */
 int mia_prefill_layer_typed(float *X, const mia_layer_weights_typed *lw, const float *theta_inv,
                             uint16_t *k_layer, uint16_t *v_layer, int dim, int hidden,
                             int n_heads, int n_kv_heads, float eps, int max_seq, int start_pos,

@@ -1,6 +1,6 @@
 """The Q4_0 GEMM tile layout of include/miattn.h (mia_q4_0_pack_gemm), restated
 with numpy index arithmetic, and the kernel's operand formation from it
-(q4_gemm_wide_kernel, tile layout) emulated on the CPU."""
+(gemm_kernel, tile layout) emulated on the CPU."""
 
 import numpy as np
 

@@ -477,3 +477,35 @@ def test_prefill_layer_typed_all_q4_0_is_prefill_layer():
     assert np.array_equal(got, dX.download(X.shape, np.float32))
     assert np.array_equal(kc_g, dkc.download(kc.shape, np.uint16))
     assert np.array_equal(vc_g, dvc.download(vc.shape, np.uint16))
+
+
+@pytest.mark.parametrize("t", [O.TYPE_Q4_0, O.TYPE_Q4_K, O.TYPE_Q6_K, O.TYPE_F16, O.TYPE_F32])
+@pytest.mark.parametrize("S,N,K", [
+    (1, 328, 512),      # one token; 8 rows in the last workgroup's second wave
+    (33, 264, 1024),    # one past the 32-token tile
+    (65, 40, 2816),     # one past 64; fewer rows than a wave has; K split unevenly
+    (129, 520, 512),    # one past 128
+    (300, 4096, 512),   # unsplit, several tiles each way
+])
+def test_gemm_tile_edges(t, S, N, K):
+    # Every weight source around the edges of its token and row tiles and of
+    # the K split, against float64 within the row bound of fp32 sums.
+    G.say(f"gemm tile edges {NAMES[t]} S={S} {N}x{K}")
+    g = np.random.default_rng(7 * S + N + K + t)
+    W = O.make_typed(g, t, N, K, d_scale=0.07)
+    X = g.standard_normal((S, K)).astype(np.float32)
+    got = gpu_gemm(W, t, X, N, K)
+    Wd = O.dequant_typed(W, t, N, K).astype(np.float64)
+    _assert_close(got, X.astype(np.float64) @ Wd.T, _bound(Wd, X), f"gemm edges {NAMES[t]}")
+
+
+@pytest.mark.parametrize("t,K", [(O.TYPE_F16, 96), (O.TYPE_F32, 160), (O.TYPE_F16, 32)])
+def test_gemm_odd_k_blocks(t, K):
+    # in_dim a multiple of 32 only: stages of 32 K values, an odd number of them
+    G.say(f"gemm odd K {NAMES[t]} K={K}")
+    g = np.random.default_rng(K)
+    W = O.make_typed(g, t, 70, K)
+    X = g.standard_normal((37, K)).astype(np.float32)
+    got = gpu_gemm(W, t, X, 70, K)
+    Wd = O.dequant_typed(W, t, 70, K).astype(np.float64)
+    _assert_close(got, X.astype(np.float64) @ Wd.T, _bound(Wd, X), f"gemm odd K {NAMES[t]}")
