@@ -33,6 +33,17 @@ constexpr int kMaxSeq = 1 << 22;  // ring capacity limit; in-layer offsets are 6
 // token takes its slot by scanning them (S^2 / 2 reads); longer chunks use a
 // per-slot area instead (one more launch, linear in S).
 constexpr int kChunkScanMax = 64;
+// mia_attention_chunk, mia_attention_positions: up to this many tokens go
+// through the decode kernel, each reading its own window; more through the flash
+// kernel, whose row tiles share the keys among 8 tokens.  Us a layer, decode
+// then flash kernel (rotation of K included, 8 kv heads):
+//   tokens   after 256 keys   1024          4064          8000
+//        4   11.1   11.6      12.1   17.2   14.9   20.3   18.9   23.9
+//        8   12.5   11.4      13.8   17.6   19.8   20.5   27.2   23.7
+//       12   17.7   11.7      21.8   17.7   36.1   21.1   54.6   24.7
+//       32    9.8   11.5      15.7   17.7   37.2   22.0   64.9   26.2
+//       64   15.1   11.7      27.3   19.2   70.3   24.0  125.6   32.4
+constexpr int kChunkFew = 8;
 // The K and V projections of layers of other weight types (hipBLASLt): workspace
 // size, algorithms timed on a shape's first call, shapes remembered.
 constexpr size_t kLtWorkspace = size_t(64) << 20;
@@ -63,6 +74,8 @@ struct DevCtx {
   size_t split_work_bytes = 0;
   int *owner = nullptr;  // long chunks of mia_attention_chunk: last token per ring slot, -1 at rest
   int owner_slots = 0;
+  int *arrive = nullptr;  // queries at positions of their own: splits done per row tile, 0 at rest
+  int arrive_tiles = 0;
   // hipBLASLt: handle and workspace created on first use, the algorithm of
   // each shape picked on its first call (lt_gemm), operands and products
   hipblasLtHandle_t lt = nullptr;
@@ -155,6 +168,19 @@ int ensure_owner(DevCtx *c, int slots) {
     HIP_TRY(hipMalloc((void **)&c->owner, (size_t)slots * sizeof(int)));
     HIP_TRY(hipMemset(c->owner, 0xFF, (size_t)slots * sizeof(int)));  // -1 everywhere
     c->owner_slots = slots;
+  }
+  return MIA_OK;
+}
+
+int ensure_arrive(DevCtx *c, int tiles) {
+  if (tiles > c->arrive_tiles) {
+    HIP_TRY(hipDeviceSynchronize());
+    if (c->arrive) HIP_TRY(hipFree(c->arrive));
+    c->arrive = nullptr;
+    c->arrive_tiles = 0;
+    HIP_TRY(hipMalloc((void **)&c->arrive, (size_t)tiles * sizeof(int)));
+    HIP_TRY(hipMemset(c->arrive, 0, (size_t)tiles * sizeof(int)));
+    c->arrive_tiles = tiles;
   }
   return MIA_OK;
 }
@@ -453,10 +479,42 @@ int decode_impl(const float *q, const float *k, const float *v, const float *the
 }
 
 // S tokens at their own positions (device int32 [S]) over the ring as it
-// stands, through the decode kernel batched over tokens; theta_inv set: Q is
-// raw and rotated in-kernel.  Every token takes the same chunk count, planned
+// stands; rope_cs set: Q is raw and rotated in-kernel.
+int positions_impl(DevCtx *c, const float *Q, const float *rope_cs, const int *positions,
+                   const uint16_t *k_layer, const uint16_t *v_layer, float *out, int n_kv,
+                   int max_seq, int S, hipStream_t s) {
+  mia::FlashParams p{};
+  int rt = 0;
+  mia::flash_positions_plan(S, n_kv, kG, max_seq, c->num_cus, &p.n_rtiles, &p.nsplit, &rt);
+  p.Q = Q;
+  p.rope_cs = rope_cs;
+  p.positions = positions;
+  p.kc = reinterpret_cast<const _Float16 *>(k_layer);
+  p.vc = reinterpret_cast<const _Float16 *>(v_layer);
+  p.out = out;
+  p.S = S;
+  p.n_kv = n_kv;
+  p.max_seq = max_seq;
+  p.qscale = qscale_log2();
+  if (p.nsplit > 1) {
+    const size_t ntile = (size_t)n_kv * p.n_rtiles;
+    if (int rc = ensure_scratch(c, mia::flash_scratch_bytes(n_kv, p.n_rtiles, p.nsplit, rt)))
+      return rc;
+    if (int rc = ensure_arrive(c, (int)ntile)) return rc;
+    p.part_o = reinterpret_cast<float *>(c->split);
+    p.part_ml = p.part_o + ntile * p.nsplit * rt * kHD;
+    p.arrive = c->arrive;
+  }
+  hipEvent_t ev0, ev1;
+  if (int rc = prof_pair(c, 0, &ev0, &ev1)) return rc;
+  HIP_TRY(mia::launch_flash_positions(p, kG, s, ev0, ev1));
+  return MIA_OK;
+}
+
+// The same for few tokens, through the decode kernel batched over tokens;
+// theta_inv set: Q is raw and rotated in-kernel.  Every token takes the same chunk count, planned
 // for the longest possible window (max_seq).
-int positions_impl(DevCtx *c, const float *Q, const float *theta_inv, const int *positions,
+int positions_few_impl(DevCtx *c, const float *Q, const float *theta_inv, const int *positions,
                    const uint16_t *k_layer, const uint16_t *v_layer, float *out, int n_kv,
                    int max_seq, int S, hipStream_t s) {
   mia::DecodeParams p{};
@@ -787,6 +845,11 @@ int mia_init(int device) {
   HIP_TRY(mia::prepare_gemm());
   HIP_TRY(hipGetSymbolAddress(&c.noalloc, HIP_SYMBOL(scratch)));
   HIP_TRY(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
+  // Scratch of mia_attention_chunk and mia_attention_positions up to
+  // kChunkScanMax tokens, so that their first call may be captured.
+  if (int rc = ensure_work(&c, (size_t)kChunkScanMax * kHD * sizeof(float))) return rc;
+  if (int rc = ensure_scratch(&c, mia::flash_positions_scratch(c.num_cus))) return rc;
+  if (int rc = ensure_arrive(&c, c.num_cus)) return rc;
   c.ready = true;
   return MIA_OK;
 }
@@ -1059,8 +1122,9 @@ int mia_attention_positions(const float *Q, float *out, const uint16_t *k_layer,
   if (int rc = check_shape(n_heads, n_kv_heads, hd, max_seq)) return rc;
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
-  return positions_impl(c, Q, nullptr, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S,
-                        pick_stream(c, stream));
+  return (S <= kChunkFew ? positions_few_impl : positions_impl)(
+      c, Q, nullptr, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S,
+      pick_stream(c, stream));
 }
 
 int mia_attention_chunk(const float *Q, const float *K, const float *V, const int *positions,
@@ -1084,12 +1148,18 @@ int mia_attention_chunk(const float *Q, const float *K, const float *V, const in
     if (int rc = ensure_owner(c, max_seq)) return rc;
     owner = c->owner;
   }
+  // (the rotation also leaves the (cos, sin) table from which the flash kernel
+  // rotates Q)
+  if (int rc = ensure_work(c, (size_t)S * kHD * sizeof(float))) return rc;
+  float *cs = reinterpret_cast<float *>(c->work);
   HIP_TRY(mia::launch_rope_kv_positions(K, V, theta_inv, positions, S, n_kv_heads,
                                         reinterpret_cast<_Float16 *>(k_layer),
                                         reinterpret_cast<_Float16 *>(v_layer), max_seq, owner,
-                                        s));
-  return positions_impl(c, Q, theta_inv, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S,
-                        s);
+                                        cs, s));
+  if (S <= kChunkFew)
+    return positions_few_impl(c, Q, theta_inv, positions, k_layer, v_layer, out, n_kv_heads,
+                              max_seq, S, s);
+  return positions_impl(c, Q, cs, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S, s);
 }
 
 int mia_attention_step(const float *Q, const float *K, const float *V, const float *theta_inv,

@@ -128,14 +128,33 @@ __global__ void slot_claim_kernel(const int *positions, int S, int max_seq, int 
 __global__ void __launch_bounds__(128)
     rope_kv_positions_kernel(const float *K, const float *V, const float *theta_inv,
                              const int *positions, int S, int n_kv, _Float16 *kc, _Float16 *vc,
-                             int max_seq, int *owner) {
+                             int max_seq, int *owner, float *cs_out) {
   __shared__ float2 cs[HD / 2];
   __shared__ int overwritten;
   const int t = blockIdx.x;
   const int tid = threadIdx.x;
   const int pos = positions[t];
-  if (pos < 0) return;  // no slot (the attention gives such a token a zero row)
+  if (pos < 0) {  // no slot (the attention gives such a token a zero row)
+    if (tid < HD / 2)
+      *reinterpret_cast<float2 *>(cs_out + (size_t)t * HD + 2 * tid) = make_float2(1.f, 0.f);
+    return;
+  }
   const int slot = pos % max_seq;
+  const int kv_dim = n_kv * HD;
+  const int n_items = n_kv * (HD / 8);
+  // (the K/V loads of the thread's first item come before the scan and the
+  // angles, as in rope_kv_f16_kernel)
+  f4 k0 = {}, k1 = {}, v0 = {}, v1 = {};
+  auto load = [&](int c) {
+    const int e0 = (c >> 4) * HD + 8 * (c & 15);
+    const f4 *ks = reinterpret_cast<const f4 *>(K + (size_t)t * kv_dim + e0);
+    const f4 *vs = reinterpret_cast<const f4 *>(V + (size_t)t * kv_dim + e0);
+    k0 = ks[0];
+    k1 = ks[1];
+    v0 = vs[0];
+    v1 = vs[1];
+  };
+  if (tid < n_items) load(tid);
   if (owner != nullptr) {
     if (tid == 0) {
       const int last = owner[slot];
@@ -155,15 +174,13 @@ __global__ void __launch_bounds__(128)
     float sn, c;
     sincosf(ang, &sn, &c);
     cs[tid] = make_float2(c, sn);
+    *reinterpret_cast<float2 *>(cs_out + (size_t)t * HD + 2 * tid) = cs[tid];
   }
   __syncthreads();
   if (overwritten) return;  // workgroup-uniform
-  const int kv_dim = n_kv * HD;
-  for (int c = tid; c < n_kv * (HD / 8); c += blockDim.x) {
+  for (int c = tid; c < n_items; c += blockDim.x) {
     const int e0 = (c >> 4) * HD + 8 * (c & 15);
-    const f4 *ks = reinterpret_cast<const f4 *>(K + (size_t)t * kv_dim + e0);
-    const f4 *vs = reinterpret_cast<const f4 *>(V + (size_t)t * kv_dim + e0);
-    const f4 k0 = ks[0], k1 = ks[1], v0 = vs[0], v1 = vs[1];
+    if (c != tid) load(c);
     float kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
     const int p0 = 4 * (c & 15);
 #pragma unroll
@@ -290,7 +307,8 @@ hipError_t launch_kv_write(_Float16 *kc, _Float16 *vc, const float *K, const flo
 
 hipError_t launch_rope_kv_positions(const float *K, const float *V, const float *theta_inv,
                                     const int *positions, int S, int n_kv, _Float16 *kc,
-                                    _Float16 *vc, int max_seq, int *owner, hipStream_t s) {
+                                    _Float16 *vc, int max_seq, int *owner, float *cs_out,
+                                    hipStream_t s) {
   if (S <= 0) return hipSuccess;
   if (owner != nullptr) {
     hipLaunchKernelGGL(slot_claim_kernel, dim3((S + 255) / 256), dim3(256), 0, s, positions, S,
@@ -299,7 +317,7 @@ hipError_t launch_rope_kv_positions(const float *K, const float *V, const float 
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(rope_kv_positions_kernel, dim3(S), dim3(128), 0, s, K, V, theta_inv,
-                     positions, S, n_kv, kc, vc, max_seq, owner);
+                     positions, S, n_kv, kc, vc, max_seq, owner, cs_out);
   return hipGetLastError();
 }
 

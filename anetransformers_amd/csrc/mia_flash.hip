@@ -45,6 +45,7 @@
 // kernel wrote.  Masks are applied only to tiles that cross a window edge.
 // Very long key ranges over few rows are also split over workgroups and merged
 // by flash_merge_kernel.
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 
@@ -57,6 +58,15 @@ namespace {
 
 constexpr int kKT = 32;     // keys per tile
 constexpr int kWaves = 4;   // key groups per workgroup, one wave each
+// Queries at positions of their own.  A split takes 640 keys or more (five
+// tiles a wave, 2.5 us: half of what merging costs; splits of 512 keys took
+// 16.9 us instead of 15.4 for 32 queries after 800 keys, splits of 128 keys
+// 19 instead of 17.7 after 1024), and a row tile at most eight splits (16: 23.5
+// us, 8: 20.1, 8 queries after 4064 keys).  32-row tiles up to where 64-row
+// tiles fill the device (8 kv heads) without splits.
+constexpr int kPosSplitKeys = 640;
+constexpr int kPosMaxSplits = 8;
+constexpr int kPosWideQueries = 512;
 
 // K/V/Q tiles live in LDS unpadded, one 256 B row per key (or query row),
 // with the 16-byte chunk c of row r stored at chunk c ^ swz(r): 16 rows read
@@ -334,6 +344,157 @@ __device__ __forceinline__ void pv_drain_all(f16v (&o)[NB][4]) {
 __device__ __forceinline__ float half_swap_max(float m) { return fmaxf(m, __shfl_xor(m, 32)); }
 __device__ __forceinline__ float half_swap_sum(float x) { return x + __shfl_xor(x, 32); }
 
+// Wave-uniform maximum.
+__device__ __forceinline__ int wave_max_int(int v) {
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) v = max(v, __shfl_xor(v, d));
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+// Partial results that another workgroup of the same launch reads: stores past
+// this XCD's L2 and loads past it (device scope, 8 bytes each).  A release
+// fence instead writes the whole L2 back, once per wave: S 32 after 4064 keys
+// took 48 us with fences, 23 with these.
+typedef unsigned long long u64;
+__device__ __forceinline__ void store_shared2(float *p, float a, float b) {
+  __hip_atomic_store(reinterpret_cast<u64 *>(p), __builtin_bit_cast(u64, (f2){a, b}),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f2 load_shared2(const float *p) {
+  return __builtin_bit_cast(f2, __hip_atomic_load(reinterpret_cast<const u64 *>(p), __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// The rows of a POS workgroup one by one in fp32, over the keys of each row
+// alone: a wave per row, two dims per lane.  In the tile loop a key past a
+// row's position has weight 0 in that row, which an infinite or NaN value there
+// turns into NaN; a workgroup with such a result comes here, so that a row
+// depends on its own window only.
+template <int NB>
+__device__ __forceinline__ void rows_alone(const FlashParams &p, int kvh, int tile_id, int row0,
+                                           int split, int n_splits, int ks, int ke) {
+  const int lane = threadIdx.x & 63;
+  const size_t kv_dim = (size_t)p.n_kv * HD;
+  for (int rl = threadIdx.x >> 6; rl < 32 * NB; rl += kWaves) {
+    const int t = (row0 + rl) >> 2, g = (row0 + rl) & 3;
+    if (t >= p.S) continue;
+    const size_t at = ((size_t)t * p.n_kv * 4 + kvh * 4 + g) * HD + 2 * lane;
+    const float2 q = *reinterpret_cast<const float2 *>(p.Q + at);
+    float q0 = q.x, q1 = q.y;
+    if (p.rope_cs != nullptr) {
+      const float2 cs = *reinterpret_cast<const float2 *>(p.rope_cs + (size_t)t * HD + 2 * lane);
+      rope_pair(q0, q1, cs.x, cs.y);
+    }
+    q0 *= p.qscale;
+    q1 *= p.qscale;
+    float m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
+    const int end = min(min(p.positions[t], p.max_seq - 1), ke - 1);
+    for (int k = ks; k <= end; ++k) {
+      const size_t off = (size_t)k * kv_dim + kvh * HD + 2 * lane;
+      const float s = wave_sum(q0 * (float)p.kc[off] + q1 * (float)p.kc[off + 1]);
+      const float mn = fmaxf(m, s);
+      const float a = m == -INFINITY ? 0.f : fast_exp2(m - mn);
+      const float w = s == -INFINITY ? 0.f : fast_exp2(s - mn);
+      m = mn;
+      l = l * a + w;
+      o0 = o0 * a + w * (float)p.vc[off];
+      o1 = o1 * a + w * (float)p.vc[off + 1];
+    }
+    float *dst = p.out + at;
+    if (n_splits == 1) {
+      const float inv = l == 0.f ? 0.f : 1.0f / l;
+      o0 *= inv;
+      o1 *= inv;
+    } else {
+      const size_t row = ((size_t)tile_id * p.nsplit + split) * (32 * NB) + rl;
+      dst = p.part_o + row * HD + 2 * lane;
+      if (lane == 0) store_shared2(p.part_ml + row * 2, m, l);
+    }
+    store_shared2(dst, o0, o1);
+  }
+}
+
+// Merge of the splits of a POS row tile by the workgroup that finishes it:
+// every workgroup counts itself in once its partials have arrived; the one that completes the count puts it back to zero and merges.  First
+// one thread per row turns the splits' (max, sum) into weights in LDS, then
+// each thread sums 4 dims of RT / 8 rows; the first splits' loads are issued
+// ahead of the weights.
+template <int NB>
+__device__ __forceinline__ void merge_last_split(const FlashParams &p, char *smem, int tile_id,
+                                                 int row0, int n_splits) {
+  constexpr int RT = 32 * NB;
+  float *const wt = reinterpret_cast<float *>(smem);  // [n_splits][RT]
+  int *const last = reinterpret_cast<int *>(wt + kPosMaxSplits * RT);
+  const int tid = threadIdx.x;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials
+  __syncthreads();  // (also: every read of LDS by the merge of the waves)
+  if (tid == 0) {
+    const int n = __hip_atomic_fetch_add(p.arrive + tile_id, 1, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    *last = n == n_splits - 1;
+    if (n == n_splits - 1)
+      __hip_atomic_store(p.arrive + tile_id, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (*last == 0) return;  // whole workgroup
+  const size_t base = (size_t)tile_id * p.nsplit * RT;
+  const int dim = 4 * (tid & 31), r0 = tid >> 5;
+  constexpr int kAhead = NB == 1 ? 4 : 2;  // splits whose loads are in flight
+  f4 x[kAhead][RT / 8];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k)
+#pragma unroll
+      for (int j = 0; j < RT / 8; ++j) {
+        const float *src =
+            p.part_o + (base + (size_t)min(k0 + k, n_splits - 1) * RT + r0 + 8 * j) * HD + dim;
+        const f2 a = load_shared2(src), b = load_shared2(src + 2);
+        x[k][j] = (f4){a.x, a.y, b.x, b.y};
+      }
+  };
+  load(0);
+  if (tid < RT) {
+    f2 ml[kPosMaxSplits];
+    float M = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < kPosMaxSplits; ++k) {
+      ml[k] = (f2){-INFINITY, 0.f};
+      if (k < n_splits) ml[k] = load_shared2(p.part_ml + (base + (size_t)k * RT + tid) * 2);
+      M = fmaxf(M, ml[k].x);
+    }
+    float l = 0.f;
+#pragma unroll
+    for (int k = 0; k < kPosMaxSplits; ++k) {
+      const float e = ml[k].x == -INFINITY ? 0.f : fast_exp2(ml[k].x - M);
+      l = __builtin_fmaf(e, ml[k].y, l);
+      ml[k].x = e;
+    }
+    const float inv = l == 0.f ? 0.f : 1.0f / l;
+#pragma unroll
+    for (int k = 0; k < kPosMaxSplits; ++k)
+      if (k < n_splits) wt[k * RT + tid] = ml[k].x * inv;
+  }
+  __syncthreads();
+  f4 acc[RT / 8];
+#pragma unroll
+  for (int j = 0; j < RT / 8; ++j) acc[j] = (f4){0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < n_splits; k0 += kAhead) {
+    if (k0 > 0) load(k0);
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k)
+#pragma unroll
+      for (int j = 0; j < RT / 8; ++j)
+        if (k0 + k < n_splits) acc[j] += wt[(k0 + k) * RT + r0 + 8 * j] * x[k][j];
+  }
+  const int kvh = tile_id / p.n_rtiles;
+#pragma unroll
+  for (int j = 0; j < RT / 8; ++j) {
+    const int row = row0 + r0 + 8 * j, t = row >> 2, g = row & 3;
+    if (t < p.S)
+      *reinterpret_cast<f4 *>(p.out + ((size_t)t * p.n_kv * 4 + kvh * 4 + g) * HD + dim) = acc[j];
+  }
+}
+
 // FAST: no staged rows.  The keys are then the ring's slots as they stand:
 // the window of position p, min(p + 1, max_seq) positions, is the slots 0 ..
 // min(p, max_seq - 1) whatever the ring's start, and the order of a softmax
@@ -344,8 +505,22 @@ __device__ __forceinline__ float half_swap_sum(float x) { return x + __shfl_xor(
 // masked (a range that ends before key 32 repeats its last key instead).  The
 // generic kernel has wrapped windows next to staged rows, with per-lane
 // addresses on the tiles that need them.
-template <int NB, bool FAST>
+//
+// POS (with FAST): query t at p.positions[t] (device memory, any order; a
+// negative position has no keys and gives a zero row) instead of start_pos +
+// t.  Windows over slots need no order of the positions: a row tile walks the
+// keys up to its largest position, and every row masks by its own.  The host
+// does not know how long the windows are, so the split is made here: the
+// launch has p.nsplit workgroups per row tile, the tile's keys are dealt in
+// splits of at least kPosSplitKeys, workgroups beyond them end at once, and
+// the last workgroup of a tile to finish merges its splits (p.arrive counts
+// them): a merge launch would cost the many short windows, which are one
+// split, 3 us for nothing.  What bounds it is latency: 4 us of the kernel are
+// its start and end, the merge of splits takes 4 to 5 us more, and a 32-key
+// tile of a wave 0.5 us.
+template <int NB, bool FAST, bool POS>
 __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
+  static_assert(FAST || !POS, "positions are windows over slots");
   using L = Lay<NB>;
   constexpr int RT = 32 * NB;  // rows per workgroup
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -367,11 +542,54 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   // Key range of the workgroup (one split), then of this wave.
   const int tq0 = row0 >> 2;
   const int tq1 = min(tq0 + RT / 4 - 1, p.S - 1);
+  const bool rope = p.rope_cs != nullptr;
+  const unsigned qstage = lds_addr(lds + (w * 4 + 3) * L::kTileHalfs);  // V1's buffer
+  const unsigned csstage =
+      lds_addr(lds + (L::kBufBytes + L::kQBytes + L::kMLBytes) / 2) + (unsigned)w * 1024u * NB;
+  const int wq0 = tq0 + 2 * NB * w;  // first query of this wave's rows
+  auto issue_q = [&] {
+#pragma unroll
+    for (int j = 0; j < 4 * NB; ++j) {  // query j/2, heads 2(j&1) .. +1
+      const int tq = min(wq0 + (j >> 1), p.S - 1);
+      dma16(p.Q + (size_t)tq * dim_model + (size_t)(kvh * 4 + 2 * (j & 1)) * HD + 4 * lane,
+            qstage + 1024u * j);
+    }
+    if (rope) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {  // queries 2j, 2j+1 of the wave
+        const int tq = min(wq0 + 2 * j + (lane >> 5), p.S - 1);
+        dma16(p.rope_cs + (size_t)tq * HD + 4 * (lane & 31), csstage + 1024u * j);
+      }
+    }
+  };
   const int klo = FAST ? 0 : window_lo(p.start_pos + tq0, p.max_seq);
   const int kcap = FAST ? p.max_seq - 1 : INT_MAX;  // the last key there is
-  const int khi = min(p.start_pos + tq1, kcap);
-  const int ks = klo + split * p.split_keys;
-  const int ke = min(ks + p.split_keys, khi + 1);
+  // POS: the row's last slot, -1 for none
+  int pos_hi[NB];
+  int khi, split_keys = p.split_keys, n_splits = p.nsplit;
+  if constexpr (POS) {
+    issue_q();  // (their latency and the positions' pass together)
+    int top = -1;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int pt = p.positions[min((row0 + 32 * b + col) >> 2, p.S - 1)];
+      pos_hi[b] = max(min(pt, kcap), -1);
+      top = max(top, pos_hi[b]);
+    }
+    khi = wave_max_int(top);
+    // (readfirstlane: the divisions leave their results in VGPRs)
+    n_splits = __builtin_amdgcn_readfirstlane(max(1, min(p.nsplit, (khi + 1) / kPosSplitKeys)));
+    split_keys = __builtin_amdgcn_readfirstlane((khi + n_splits) / n_splits);  // (khi < 2^22)
+    split_keys = max(kKT, (split_keys + kKT - 1) / kKT * kKT);
+    if (split >= n_splits) {  // whole workgroup
+      wait_vmcnt<0>();
+      return;
+    }
+  } else {
+    khi = min(p.start_pos + tq1, kcap);
+  }
+  const int ks = klo + split * split_keys;
+  const int ke = min(ks + split_keys, khi + 1);
   const int nt = ke > ks ? (ke - ks + kKT - 1) / kKT : 0;
   // Key groups interleaved by tile: wave w takes tiles w, w + 4, w + 8, ...
   // of the range.  The waves then share the masked tiles at the causal edge
@@ -390,6 +608,14 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   for (int b = 0; b < NB; ++b) {
     const int t = (row0 + 32 * b + col) >> 2;
     valid[b] = t < p.S;
+    if constexpr (POS) {
+      valid[b] = valid[b] && pos_hi[b] >= 0;
+      lo_t[b] = lo_max[b] = 0;
+      hi_t[b] = pos_hi[b];
+      hi_min[b] = -wave_max_int(-pos_hi[b]);  // (-1: the block is masked)
+      bfull[b] = ((row0 + 32 * b + 31) >> 2) < p.S;
+      continue;
+    }
     const int pos_t = p.start_pos + (valid[b] ? t : p.S - 1);
     lo_t[b] = FAST ? 0 : window_lo(pos_t, p.max_seq);
     hi_t[b] = min(pos_t, kcap);
@@ -511,27 +737,10 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   // written by the K rotation, mistral_model.h:87-105) and the score scale
   // folded in; rows past the last query are zero.  Each wave stages its own
   // 8 NB rows (queries 2 NB w ..) as fp32, and their (cos, sin) rows, with
-  // direct loads issued before the first tiles' (the Q rows then wait for
-  // nothing issued after them); V1's buffer holds the rows until V1 is loaded.
+  // direct loads issued before the first tiles' (issue_q; the Q rows then wait
+  // for nothing issued after them); V1's buffer holds the rows until V1 is loaded.
   lds_half *qs = lds + L::kBufBytes / 2;
-  const bool rope = p.rope_cs != nullptr;
-  const unsigned qstage = kt_a[0] + 3u * L::kTileHalfs * 2u;  // == vt_a[1]
-  const unsigned csstage =
-      lds_addr(lds + (L::kBufBytes + L::kQBytes + L::kMLBytes) / 2) + (unsigned)w * 1024u * NB;
-  const int wq0 = tq0 + 2 * NB * w;  // first query of this wave's rows
-#pragma unroll
-  for (int j = 0; j < 4 * NB; ++j) {  // query j/2, heads 2(j&1) .. +1
-    const int tq = min(wq0 + (j >> 1), p.S - 1);
-    dma16(p.Q + (size_t)tq * dim_model + (size_t)(kvh * 4 + 2 * (j & 1)) * HD + 4 * lane,
-          qstage + 1024u * j);
-  }
-  if (rope) {
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {  // queries 2j, 2j+1 of the wave
-      const int tq = min(wq0 + 2 * j + (lane >> 5), p.S - 1);
-      dma16(p.rope_cs + (size_t)tq * HD + 4 * (lane & 31), csstage + 1024u * j);
-    }
-  }
+  if constexpr (!POS) issue_q();
   issue_first_tiles();
   // the Q rows are in once at most the tile loads issued after them are pending
   if (g_count > 1) wait_vmcnt<24>();
@@ -1268,6 +1477,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   __syncthreads();
 
   const size_t tile_id = (size_t)kvh * p.n_rtiles + rtile;
+  float finite = 0.f;  // POS: 0, or NaN once a result is not finite
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     f2 mlw[kWaves];
@@ -1298,10 +1508,16 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
         for (int k = 0; k < kWaves; ++k)
           if (k != db) acc[q] += *(lds_f4 *)mg_at(k, b, db, q) * e[k];
       }
+      if constexpr (POS) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) finite = __builtin_fmaf(acc[q][i], 0.f, finite);
+      }
       if (t < p.S) {
         // dims 32*db + 8*q + 4*half .. +4 (the accumulator's dim order)
-        if (p.nsplit == 1) {
-          const float inv = 1.0f / Ls;
+        if (n_splits == 1) {
+          const float inv = POS && Ls == 0.f ? 0.f : 1.0f / Ls;  // (no keys: zeros)
           float *dst = p.out + (size_t)t * dim_model + (size_t)(kvh * 4 + g) * HD + 32 * db + 4 * half;
 #pragma unroll
           for (int q = 0; q < 4; ++q) *reinterpret_cast<f4 *>(dst + 8 * q) = acc[q] * inv;
@@ -1309,12 +1525,26 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
           const size_t pidx = (tile_id * p.nsplit + split) * RT + rl;
           float *dst = p.part_o + pidx * HD + 32 * db + 4 * half;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) *reinterpret_cast<f4 *>(dst + 8 * q) = acc[q];
-          if (db == 0 && half == 0)
-            *reinterpret_cast<float2 *>(p.part_ml + pidx * 2) = make_float2(M, Ls);
+          for (int q = 0; q < 4; ++q) {
+            if constexpr (POS) {
+              store_shared2(dst + 8 * q, acc[q][0], acc[q][1]);
+              store_shared2(dst + 8 * q + 2, acc[q][2], acc[q][3]);
+            } else {
+              *reinterpret_cast<f4 *>(dst + 8 * q) = acc[q];
+            }
+          }
+          if (db == 0 && half == 0) {
+            if constexpr (POS) store_shared2(p.part_ml + pidx * 2, M, Ls);
+            else *reinterpret_cast<float2 *>(p.part_ml + pidx * 2) = make_float2(M, Ls);
+          }
         }
       }
     }
+  }
+  if constexpr (POS) {
+    if (__syncthreads_or(finite != 0.f))
+      rows_alone<NB>(p, kvh, (int)tile_id, row0, split, n_splits, ks, ke);
+    if (n_splits > 1) merge_last_split<NB>(p, smem, (int)tile_id, row0, n_splits);
   }
 }
 
@@ -1402,9 +1632,9 @@ __global__ void __launch_bounds__(256) flash_merge_kernel(FlashParams p, int rt)
   }
 }
 
-template <int NB, bool FAST>
+template <int NB, bool FAST, bool POS>
 hipError_t set_lds_limit() {
-  return hipFuncSetAttribute((const void *)flash_kernel<NB, FAST>,
+  return hipFuncSetAttribute((const void *)flash_kernel<NB, FAST, POS>,
                              hipFuncAttributeMaxDynamicSharedMemorySize, Lay<NB>::kBytes);
 }
 
@@ -1415,20 +1645,22 @@ hipError_t launch_variant(const FlashParams &p, hipStream_t s, hipEvent_t ev0, h
   using L = Lay<NB>;
   dim3 grid(p.n_kv * p.n_rtiles * p.nsplit);
   if (p.kstage == nullptr && p.vstage == nullptr)
-    hipExtLaunchKernelGGL((flash_kernel<NB, true>), grid, dim3(256), L::kBytes, s, ev0, ev1, 0, p);
+    hipExtLaunchKernelGGL((flash_kernel<NB, true, false>), grid, dim3(256), L::kBytes, s, ev0, ev1, 0, p);
   else
-    hipExtLaunchKernelGGL((flash_kernel<NB, false>), grid, dim3(256), L::kBytes, s, ev0, ev1, 0,
-                          p);
+    hipExtLaunchKernelGGL((flash_kernel<NB, false, false>), grid, dim3(256), L::kBytes, s, ev0, ev1,
+                          0, p);
   return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t prepare_flash() {
-  hipError_t e = set_lds_limit<1, false>();
-  if (e == hipSuccess) e = set_lds_limit<2, false>();
-  if (e == hipSuccess) e = set_lds_limit<1, true>();
-  return e != hipSuccess ? e : set_lds_limit<2, true>();
+  hipError_t e = set_lds_limit<1, false, false>();
+  if (e == hipSuccess) e = set_lds_limit<2, false, false>();
+  if (e == hipSuccess) e = set_lds_limit<1, true, false>();
+  if (e == hipSuccess) e = set_lds_limit<2, true, false>();
+  if (e == hipSuccess) e = set_lds_limit<1, true, true>();
+  return e != hipSuccess ? e : set_lds_limit<2, true, true>();
 }
 
 size_t flash_scratch_bytes(int n_kv, int n_rtiles, int nsplit, int rows_per_tile) {
@@ -1478,6 +1710,39 @@ hipError_t launch_flash(const FlashParams &p, int G, hipStream_t s, hipEvent_t e
   if (G != 4) return hipErrorInvalidValue;
   return rows_per_tile(p.S) == 32 ? launch_variant<1>(p, s, ev0, ev1)
                                   : launch_variant<2>(p, s, ev0, ev1);
+}
+
+void flash_positions_plan(int S, int n_kv, int G, int max_seq, int target_wgs, int *n_rtiles,
+                          int *nsplit, int *rows_per_tile_out) {
+  const int rt = S >= kPosWideQueries ? 64 : 32;
+  const int ntiles = (S * G + rt - 1) / rt;
+  const long tiles = (long)n_kv * ntiles;
+  long ns = (target_wgs + tiles / 2) / tiles;
+  const long longest = max_seq / kPosSplitKeys;
+  ns = std::min(ns, std::min(longest, (long)kPosMaxSplits));
+  *n_rtiles = ntiles;
+  *nsplit = ns < 1 ? 1 : (int)ns;
+  *rows_per_tile_out = rt;
+}
+
+size_t flash_positions_scratch(int target_wgs) {
+  // tiles * nsplit <= target_wgs + tiles / 2, with fewer tiles than target_wgs
+  return flash_scratch_bytes(1, 1, target_wgs + target_wgs / 2, 32);
+}
+
+hipError_t launch_flash_positions(const FlashParams &p, int G, hipStream_t s, hipEvent_t ev0,
+                                  hipEvent_t ev1) {
+  if (G != 4 || p.positions == nullptr || p.nsplit < 1 || p.nsplit > kPosMaxSplits ||
+      (p.nsplit > 1 && p.arrive == nullptr))
+    return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(p.n_kv * p.n_rtiles * p.nsplit));
+  if (p.S >= kPosWideQueries)
+    hipExtLaunchKernelGGL((flash_kernel<2, true, true>), grid, dim3(256), Lay<2>::kBytes, s, ev0,
+                          ev1, 0, p);
+  else
+    hipExtLaunchKernelGGL((flash_kernel<1, true, true>), grid, dim3(256), Lay<1>::kBytes, s, ev0,
+                          ev1, 0, p);
+  return hipGetLastError();
 }
 
 hipError_t launch_flash_merge(const FlashParams &p, hipStream_t s) {

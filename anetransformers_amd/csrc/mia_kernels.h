@@ -70,6 +70,8 @@ struct FlashParams {
   int nsplit;              // key splits per row tile
   int split_keys;          // keys per split (multiple of 64)
   float qscale;
+  const int *positions;    // launch_flash_positions: the queries' positions [S]
+  int *arrive;             // and, with nsplit > 1, a count per row tile, 0 at rest
 };
 size_t flash_scratch_bytes(int n_kv, int n_rtiles, int nsplit, int rows_per_tile);
 // Main kernel only; launch_flash_merge adds the split merge (nsplit > 1).
@@ -78,6 +80,15 @@ hipError_t launch_flash(const FlashParams &p, int G, hipStream_t s, hipEvent_t e
 hipError_t launch_flash_merge(const FlashParams &p, hipStream_t s);
 void flash_plan(int S, int n_kv, int G, int start_pos, int max_seq, bool staged, int target_wgs,
                 int *n_rtiles, int *nsplit, int *split_keys, int *rows_per_tile);
+// Queries at positions of their own (device int32 [S]) over the ring as it
+// stands, one launch with the merge of its splits in it.  The partials take
+// flash_scratch_bytes; p.start_pos, split_keys and the staged rows are unused.
+void flash_positions_plan(int S, int n_kv, int G, int max_seq, int target_wgs, int *n_rtiles,
+                          int *nsplit, int *rows_per_tile);
+// The largest scratch of a plan with 32-row tiles.
+size_t flash_positions_scratch(int target_wgs);
+hipError_t launch_flash_positions(const FlashParams &p, int G, hipStream_t s, hipEvent_t ev0,
+                                  hipEvent_t ev1);
 
 // Elementwise helpers.
 hipError_t launch_rope(float *q, float *k, int S, int start_pos, const float *theta_inv,
@@ -98,9 +109,11 @@ hipError_t launch_kv_write(_Float16 *kc, _Float16 *vc, const float *K, const flo
 // chunk takes the same slot (the reference's in-order writes leave the last).
 // owner: null (each token scans the later ones, O(S^2) reads: short chunks)
 // or an int32 [max_seq] area holding -1 everywhere, left so (linear in S).
+// cs_out receives the [S][64] (cos, sin) table of the positions.
 hipError_t launch_rope_kv_positions(const float *K, const float *V, const float *theta_inv,
                                     const int *positions, int S, int n_kv, _Float16 *kc,
-                                    _Float16 *vc, int max_seq, int *owner, hipStream_t s);
+                                    _Float16 *vc, int max_seq, int *owner, float *cs_out,
+                                    hipStream_t s);
 // Staged rows 0..S-1 -> ring slots (start_pos + t) % max_seq, for n_layers
 // layers ring_stride / stage_stride elements apart.
 hipError_t launch_commit(_Float16 *kc, _Float16 *vc, const _Float16 *kst, const _Float16 *vst,

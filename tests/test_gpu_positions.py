@@ -166,3 +166,66 @@ def test_dropin_prefill_chunk_attention_two_layers():
         assert kv.len == 332
     finally:
         lib.mia_dropin_kv_free(ctypes.byref(kv))
+
+
+# (tokens, ring, positions' span): the decode kernel up to 8 tokens, then row tiles of 8 and (from
+# 512 tokens) 16 tokens and their remainders, windows at the edges of a 32-key tile and of where
+# the keys are split
+@pytest.mark.parametrize("S,M,span", [
+    (1, 31, 29), (8, 513, 513), (9, 31, 29), (10, 33, 40), (15, 640, 640), (16, 1279, 1300),
+    (17, 1280, 1280), (9, 1281, 1281), (33, 4100, 4100), (64, 8192, 20000), (65, 2600, 2600),
+    (511, 640, 640), (512, 96, 96), (517, 1400, 1500),
+])
+def test_attention_positions_tiles_and_splits(S, M, span):
+    # unsorted positions with negative ones among them, twice (the counters that the merge of the
+    # splits uses are back at rest); error bound as every other attention test's
+    G.say(f"attention_positions S={S} M={M} span={span}")
+    lib = G.lib()
+    g = D.rng(830 + S + M)
+    kc, vc = D.ring(g, M, spike_every=256)
+    positions = g.integers(0, span, S).astype(np.int32)
+    positions[0] = span - 1
+    if S > 2:
+        positions[S // 2] = -3
+    Q = D.normal(g, (S, 4096))
+    dkc, dvc, dq, dp = DB.from_array(kc), DB.from_array(vc), DB.from_array(Q), DB.from_array(positions)
+    rows = range(S) if S < 12 else sorted({0, 1, 7, 8, S // 2, S - 2, S - 1})
+    for turn in range(2):
+        dout = DB.from_array(np.full((S, 4096), np.nan, np.float32))
+        check(lib.mia_attention_positions(dq.ptr, dout.ptr, dkc.ptr, dvc.ptr, dp.ptr, 32, 8, 128,
+                                          M, S, None), "attention_positions")
+        check(lib.mia_stream_sync(None), "sync")
+        out = dout.download((S, 4096), np.float32)
+        assert np.all(np.isfinite(out))
+        for t in rows:
+            if positions[t] < 0:
+                assert np.all(out[t] == 0.0)
+            else:
+                ref = D.gqa_decode_f64(Q[t], kc, vc, 32, 8, 128, M, int(positions[t]))
+                D.check_close(out[t], ref, what=f"turn={turn} t={t} pos={positions[t]}")
+
+
+@pytest.mark.parametrize("M", [300, 3000])
+def test_attention_positions_rows_depend_on_their_own_window_only(M):
+    # infinite and NaN values and keys past a row's position, inside the windows of rows that share
+    # its tile: the row is what it is without them
+    G.say(f"attention_positions M={M} with infinities past a position")
+    lib = G.lib()
+    g = D.rng(840 + M)
+    kc, vc = D.ring(g, M)
+    positions = np.array([M // 2 - 1, 3, M - 1, M // 2 - 7, 0, 9, 40, 77, 2, 50], np.int32)
+    kc[M // 2 + 5, :] = 0x7E00  # NaN
+    vc[M // 2, :] = 0x7C00      # inf
+    vc[M // 2 + 1, 7] = 0x7E00
+    S = len(positions)
+    Q = D.normal(g, (S, 4096))
+    dkc, dvc, dq, dp = DB.from_array(kc), DB.from_array(vc), DB.from_array(Q), DB.from_array(positions)
+    dout = DB(S * 4096 * 4)
+    check(lib.mia_attention_positions(dq.ptr, dout.ptr, dkc.ptr, dvc.ptr, dp.ptr, 32, 8, 128, M,
+                                      S, None), "attention_positions")
+    check(lib.mia_stream_sync(None), "sync")
+    out = dout.download((S, 4096), np.float32)
+    assert not np.any(np.isfinite(out[2]))
+    for t in (0, 1, 3, 4, 5, 6, 7, 8, 9):
+        ref = D.gqa_decode_f64(Q[t], kc[:M // 2], vc[:M // 2], 32, 8, 128, M // 2, int(positions[t]))
+        D.check_close(out[t], ref, what=f"t={t}")
