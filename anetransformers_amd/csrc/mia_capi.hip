@@ -44,6 +44,18 @@ constexpr int kChunkScanMax = 64;
 //       32    9.8   11.5      15.7   17.7   37.2   22.0   64.9   26.2
 //       64   15.1   11.7      27.3   19.2   70.3   24.0  125.6   32.4
 constexpr int kChunkFew = 8;
+// Unstaged steps take the same kernel where its 32-row tiles fit the device at
+// once, except kChunkFew and fewer tokens, and up to kShortOnly tokens after
+// more than kShortKeys keys (separate merge: 20.6 us, here 22.0, 16 tokens
+// after 4064 keys).  Us a layer with 64-row tiles and the merge as a launch of
+// its own, then here:
+//   tokens   after 64 keys   700           2048          6000
+//       16   12.4    9.3     16.6   14.3   18.2   18.8   21.6   22.9
+//       64   12.8    9.8     24.3   14.4   27.4   20.5   32.2   28.3
+//      128   13.5   11.1     33.8   15.5   38.9   23.8   49.1   40.1
+//      256   15.6   12.5     51.9   17.4   60.1   28.6   86.5   63.9
+constexpr int kShortOnly = 16;
+constexpr int kShortKeys = 1024;
 // The K and V projections of layers of other weight types (hipBLASLt): workspace
 // size, algorithms timed on a shape's first call, shapes remembered.
 constexpr size_t kLtWorkspace = size_t(64) << 20;
@@ -480,12 +492,15 @@ int decode_impl(const float *q, const float *k, const float *v, const float *the
 
 // S tokens at their own positions (device int32 [S]) over the ring as it
 // stands; rope_cs set: Q is raw and rotated in-kernel.
+// positions null: start_pos + t.
 int positions_impl(DevCtx *c, const float *Q, const float *rope_cs, const int *positions,
                    const uint16_t *k_layer, const uint16_t *v_layer, float *out, int n_kv,
-                   int max_seq, int S, hipStream_t s) {
+                   int max_seq, int S, hipStream_t s, int start_pos = 0) {
   mia::FlashParams p{};
   int rt = 0;
-  mia::flash_positions_plan(S, n_kv, kG, max_seq, c->num_cus, &p.n_rtiles, &p.nsplit, &rt);
+  const int longest = positions == nullptr ? (int)std::min((long)start_pos + S, (long)max_seq) : max_seq;
+  mia::flash_shared_plan(S, n_kv, kG, longest, c->num_cus, &p.n_rtiles, &p.nsplit, &rt);
+  p.start_pos = start_pos;
   p.Q = Q;
   p.rope_cs = rope_cs;
   p.positions = positions;
@@ -506,8 +521,8 @@ int positions_impl(DevCtx *c, const float *Q, const float *rope_cs, const int *p
     p.arrive = c->arrive;
   }
   hipEvent_t ev0, ev1;
-  if (int rc = prof_pair(c, 0, &ev0, &ev1)) return rc;
-  HIP_TRY(mia::launch_flash_positions(p, kG, s, ev0, ev1));
+  if (int rc = prof_pair(c, positions == nullptr ? 1 : 0, &ev0, &ev1)) return rc;
+  HIP_TRY(mia::launch_flash_shared(p, kG, s, ev0, ev1));
   return MIA_OK;
 }
 
@@ -556,6 +571,11 @@ int check_positions(const int *positions, int S) {
 int flash_impl(DevCtx *c, const float *Q, const float *rope_cs, const uint16_t *kst,
                const uint16_t *vst, const uint16_t *k_layer, const uint16_t *v_layer, float *out,
                int n_kv, int max_seq, int start_pos, int S, hipStream_t s, bool commit = false) {
+  const long keys = std::min((long)start_pos + S, (long)max_seq);
+  if (kst == nullptr && S > kChunkFew && (long)n_kv * ((S + 7) / 8) <= c->num_cus &&
+      (S > kShortOnly || keys <= kShortKeys))
+    return positions_impl(c, Q, rope_cs, nullptr, k_layer, v_layer, out, n_kv, max_seq, S, s,
+                          start_pos);
   mia::FlashParams p{};
   int rt = 0;
   mia::flash_plan(S, n_kv, kG, start_pos, max_seq, kst != nullptr, c->num_cus, &p.n_rtiles,
@@ -848,7 +868,7 @@ int mia_init(int device) {
   // Scratch of mia_attention_chunk and mia_attention_positions up to
   // kChunkScanMax tokens, so that their first call may be captured.
   if (int rc = ensure_work(&c, (size_t)kChunkScanMax * kHD * sizeof(float))) return rc;
-  if (int rc = ensure_scratch(&c, mia::flash_positions_scratch(c.num_cus))) return rc;
+  if (int rc = ensure_scratch(&c, mia::flash_shared_scratch(c.num_cus))) return rc;
   if (int rc = ensure_arrive(&c, c.num_cus)) return rc;
   c.ready = true;
   return MIA_OK;
@@ -1122,9 +1142,11 @@ int mia_attention_positions(const float *Q, float *out, const uint16_t *k_layer,
   if (int rc = check_shape(n_heads, n_kv_heads, hd, max_seq)) return rc;
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
-  return (S <= kChunkFew ? positions_few_impl : positions_impl)(
-      c, Q, nullptr, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S,
-      pick_stream(c, stream));
+  hipStream_t s = pick_stream(c, stream);
+  if (S <= kChunkFew)
+    return positions_few_impl(c, Q, nullptr, positions, k_layer, v_layer, out, n_kv_heads, max_seq,
+                              S, s);
+  return positions_impl(c, Q, nullptr, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S, s);
 }
 
 int mia_attention_chunk(const float *Q, const float *K, const float *V, const int *positions,

@@ -58,15 +58,13 @@ namespace {
 
 constexpr int kKT = 32;     // keys per tile
 constexpr int kWaves = 4;   // key groups per workgroup, one wave each
-// Queries at positions of their own.  A split takes 640 keys or more (five
+// POS launches (flash_kernel).  A split takes 640 keys or more (five
 // tiles a wave, 2.5 us: half of what merging costs; splits of 512 keys took
 // 16.9 us instead of 15.4 for 32 queries after 800 keys, splits of 128 keys
 // 19 instead of 17.7 after 1024), and a row tile at most eight splits (16: 23.5
-// us, 8: 20.1, 8 queries after 4064 keys).  32-row tiles up to where 64-row
-// tiles fill the device (8 kv heads) without splits.
+// us, 8: 20.1, 8 queries after 4064 keys).
 constexpr int kPosSplitKeys = 640;
 constexpr int kPosMaxSplits = 8;
-constexpr int kPosWideQueries = 512;
 
 // K/V/Q tiles live in LDS unpadded, one 256 B row per key (or query row),
 // with the 16-byte chunk c of row r stored at chunk c ^ swz(r): 16 rows read
@@ -344,6 +342,11 @@ __device__ __forceinline__ void pv_drain_all(f16v (&o)[NB][4]) {
 __device__ __forceinline__ float half_swap_max(float m) { return fmaxf(m, __shfl_xor(m, 32)); }
 __device__ __forceinline__ float half_swap_sum(float x) { return x + __shfl_xor(x, 32); }
 
+// Position of query t of a POS launch.
+__device__ __forceinline__ int query_pos(const FlashParams &p, int t) {
+  return p.positions != nullptr ? p.positions[t] : p.start_pos + t;
+}
+
 // Wave-uniform maximum.
 __device__ __forceinline__ int wave_max_int(int v) {
 #pragma unroll
@@ -388,7 +391,7 @@ __device__ __forceinline__ void rows_alone(const FlashParams &p, int kvh, int ti
     q0 *= p.qscale;
     q1 *= p.qscale;
     float m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
-    const int end = min(min(p.positions[t], p.max_seq - 1), ke - 1);
+    const int end = min(min(query_pos(p, t), p.max_seq - 1), ke - 1);
     for (int k = ks; k <= end; ++k) {
       const size_t off = (size_t)k * kv_dim + kvh * HD + 2 * lane;
       const float s = wave_sum(q0 * (float)p.kc[off] + q1 * (float)p.kc[off + 1]);
@@ -506,18 +509,19 @@ __device__ __forceinline__ void merge_last_split(const FlashParams &p, char *sme
 // generic kernel has wrapped windows next to staged rows, with per-lane
 // addresses on the tiles that need them.
 //
-// POS (with FAST): query t at p.positions[t] (device memory, any order; a
-// negative position has no keys and gives a zero row) instead of start_pos +
-// t.  Windows over slots need no order of the positions: a row tile walks the
-// keys up to its largest position, and every row masks by its own.  The host
-// does not know how long the windows are, so the split is made here: the
-// launch has p.nsplit workgroups per row tile, the tile's keys are dealt in
-// splits of at least kPosSplitKeys, workgroups beyond them end at once, and
-// the last workgroup of a tile to finish merges its splits (p.arrive counts
-// them): a merge launch would cost the many short windows, which are one
-// split, 3 us for nothing.  What bounds it is latency: 4 us of the kernel are
-// its start and end, the merge of splits takes 4 to 5 us more, and a 32-key
-// tile of a wave 0.5 us.
+// POS (with FAST): a position per query, p.positions[t] (device memory, any
+// order; a negative position has no keys and gives a zero row) or start_pos +
+// t, and the split and its merge in the kernel.  Windows over slots need no
+// order of the positions: a row tile walks the keys up to its largest
+// position, and every row masks by its own.  The host need not know how long
+// the windows are: the launch has p.nsplit workgroups per row tile, the tile's
+// keys are dealt in splits of at least kPosSplitKeys, workgroups beyond them
+// end at once, and the last workgroup of a tile to finish merges its splits
+// (p.arrive counts them).  A short window, one split, pays nothing for that,
+// where a merge launch takes 3 us, or far more over many rows (a workgroup per
+// row: 30 us at 256 queries).  What bounds it is latency: 4 us of the kernel are its
+// start and end, the merge of splits takes 4 to 5 us more, and a 32-key tile
+// of a wave 0.5 us.
 template <int NB, bool FAST, bool POS>
 __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   static_assert(FAST || !POS, "positions are windows over slots");
@@ -572,7 +576,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     int top = -1;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int pt = p.positions[min((row0 + 32 * b + col) >> 2, p.S - 1)];
+      const int pt = query_pos(p, min((row0 + 32 * b + col) >> 2, p.S - 1));
       pos_hi[b] = max(min(pt, kcap), -1);
       top = max(top, pos_hi[b]);
     }
@@ -1712,31 +1716,35 @@ hipError_t launch_flash(const FlashParams &p, int G, hipStream_t s, hipEvent_t e
                                   : launch_variant<2>(p, s, ev0, ev1);
 }
 
-void flash_positions_plan(int S, int n_kv, int G, int max_seq, int target_wgs, int *n_rtiles,
-                          int *nsplit, int *rows_per_tile_out) {
-  const int rt = S >= kPosWideQueries ? 64 : 32;
-  const int ntiles = (S * G + rt - 1) / rt;
-  const long tiles = (long)n_kv * ntiles;
-  long ns = (target_wgs + tiles / 2) / tiles;
-  const long longest = max_seq / kPosSplitKeys;
-  ns = std::min(ns, std::min(longest, (long)kPosMaxSplits));
+// 32-row tiles, and splits of them, up to where they fill the device; beyond,
+// 64-row tiles, which do less work per key (384 queries after 2048 keys: 40.6
+// us with 64 rows, 50.7 with 32, at one or two workgroups a CU).
+void flash_shared_plan(int S, int n_kv, int G, int longest, int target_wgs, int *n_rtiles,
+                       int *nsplit, int *rows_per_tile_out) {
+  int rt = 32;
+  int ntiles = (S * G + rt - 1) / rt;
+  if ((long)n_kv * ntiles > target_wgs) {
+    rt = 64;
+    ntiles = (S * G + rt - 1) / rt;
+  }
+  const long fill = target_wgs / ((long)n_kv * ntiles);
+  const long ns = std::min(fill, std::min((long)longest / kPosSplitKeys, (long)kPosMaxSplits));
   *n_rtiles = ntiles;
   *nsplit = ns < 1 ? 1 : (int)ns;
   *rows_per_tile_out = rt;
 }
 
-size_t flash_positions_scratch(int target_wgs) {
-  // tiles * nsplit <= target_wgs + tiles / 2, with fewer tiles than target_wgs
-  return flash_scratch_bytes(1, 1, target_wgs + target_wgs / 2, 32);
+size_t flash_shared_scratch(int target_wgs) {
+  return flash_scratch_bytes(1, 1, target_wgs, 64);  // tiles * nsplit <= target_wgs
 }
 
-hipError_t launch_flash_positions(const FlashParams &p, int G, hipStream_t s, hipEvent_t ev0,
+hipError_t launch_flash_shared(const FlashParams &p, int G, hipStream_t s, hipEvent_t ev0,
                                   hipEvent_t ev1) {
-  if (G != 4 || p.positions == nullptr || p.nsplit < 1 || p.nsplit > kPosMaxSplits ||
+  if (G != 4 || p.nsplit < 1 || p.nsplit > kPosMaxSplits ||
       (p.nsplit > 1 && p.arrive == nullptr))
     return hipErrorInvalidValue;
   const dim3 grid((unsigned)(p.n_kv * p.n_rtiles * p.nsplit));
-  if (p.S >= kPosWideQueries)
+  if (p.n_rtiles != (p.S * G + 31) / 32)
     hipExtLaunchKernelGGL((flash_kernel<2, true, true>), grid, dim3(256), Lay<2>::kBytes, s, ev0,
                           ev1, 0, p);
   else

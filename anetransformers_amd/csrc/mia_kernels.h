@@ -70,7 +70,7 @@ struct FlashParams {
   int nsplit;              // key splits per row tile
   int split_keys;          // keys per split (multiple of 64)
   float qscale;
-  const int *positions;    // launch_flash_positions: the queries' positions [S]
+  const int *positions;    // launch_flash_shared: the queries' positions [S], or null
   int *arrive;             // and, with nsplit > 1, a count per row tile, 0 at rest
 };
 size_t flash_scratch_bytes(int n_kv, int n_rtiles, int nsplit, int rows_per_tile);
@@ -80,15 +80,16 @@ hipError_t launch_flash(const FlashParams &p, int G, hipStream_t s, hipEvent_t e
 hipError_t launch_flash_merge(const FlashParams &p, hipStream_t s);
 void flash_plan(int S, int n_kv, int G, int start_pos, int max_seq, bool staged, int target_wgs,
                 int *n_rtiles, int *nsplit, int *split_keys, int *rows_per_tile);
-// Queries at positions of their own (device int32 [S]) over the ring as it
-// stands, one launch with the merge of its splits in it.  The partials take
-// flash_scratch_bytes; p.start_pos, split_keys and the staged rows are unused.
-void flash_positions_plan(int S, int n_kv, int G, int max_seq, int target_wgs, int *n_rtiles,
-                          int *nsplit, int *rows_per_tile);
-// The largest scratch of a plan with 32-row tiles.
-size_t flash_positions_scratch(int target_wgs);
-hipError_t launch_flash_positions(const FlashParams &p, int G, hipStream_t s, hipEvent_t ev0,
-                                  hipEvent_t ev1);
+// The flash kernel with the split and its merge in one launch, over the ring as
+// it stands: queries at p.positions (device int32 [S]) or, where that is null,
+// at start_pos + t.  longest: the most keys a window can have.  The partials
+// take flash_scratch_bytes; p.split_keys and the staged rows are unused.
+void flash_shared_plan(int S, int n_kv, int G, int longest, int target_wgs, int *n_rtiles,
+                       int *nsplit, int *rows_per_tile);
+// The largest scratch of a plan.
+size_t flash_shared_scratch(int target_wgs);
+hipError_t launch_flash_shared(const FlashParams &p, int G, hipStream_t s, hipEvent_t ev0,
+                               hipEvent_t ev1);
 
 // Elementwise helpers.
 hipError_t launch_rope(float *q, float *k, int S, int start_pos, const float *theta_inv,

@@ -295,3 +295,29 @@ def test_attention_batch_ring_in_slot_order(M, start, S):
         n = min(start + t + 1, M)
         exact[t] = D.gqa_decode_f64(Q[t], kc[:n], vc[:n], 32, 8, 128, n, n - 1)
     D.check_close(out, exact, what=f"slot order M={M} start={start} S={S}")
+
+
+@pytest.mark.parametrize("M,start,S", [
+    (8192, 0, 9), (8192, 1008, 16), (8192, 1009, 16),  # 8-token tiles; the merge as its own launch
+    (8192, 1260, 20), (8192, 1261, 20),                # one split, two splits
+    (8192, 7000, 17), (700, 3000, 33),                 # eight splits; a wrapped ring in one
+    (4096, 1300, 128), (4096, 1300, 129),              # two splits of every tile, none
+    (2048, 700, 256), (2048, 700, 257),                # 8-token tiles fill the device; 16-token tiles
+])
+def test_attention_batch_tiles_and_splits(M, start, S):
+    # Where the row tile, the split of the keys and its merge change; twice (the merge's counters
+    # are back at rest).
+    G.say(f"attention_batch tiles and splits M={M} start={start} S={S}")
+    g = D.rng(7 * M + start + S)
+    filled = min(start + S, M)
+    kc, vc = D.ring(g, M, filled=filled, spike_every=256)
+    kc[filled:], vc[filled:] = 0x7E00, 0x7E00
+    Q = D.normal(g, (S, 4096))
+    rows = range(S) if S < 20 else sorted({0, 1, 7, 8, S // 2, S - 2, S - 1})
+    for turn in range(2):
+        out = G.attention_batch(Q, kc, vc, M, start, S)
+        assert np.all(np.isfinite(out))
+        for t in rows:
+            n = min(start + t + 1, M)
+            exact = D.gqa_decode_f64(Q[t], kc[:n], vc[:n], 32, 8, 128, n, n - 1)
+            D.check_close(out[t], exact, what=f"turn={turn} M={M} start={start} S={S} t={t}")
