@@ -490,25 +490,33 @@ int decode_impl(const float *q, const float *k, const float *v, const float *the
   return MIA_OK;
 }
 
+void set_out_planes(mia::FlashParams &p, _Float16 *planes) {
+  if (planes == nullptr) return;
+  p.out_hi = planes;
+  p.out_lo = planes + (size_t)p.S * p.n_kv * kG * kHD;
+}
+
 // S tokens at their own positions (device int32 [S]) over the ring as it
 // stands; rope_cs set: Q is raw and rotated in-kernel.
-// positions null: start_pos + t.
+// positions null: start_pos + t.  out_planes: flash_impl's.
 int positions_impl(DevCtx *c, const float *Q, const float *rope_cs, const int *positions,
                    const uint16_t *k_layer, const uint16_t *v_layer, float *out, int n_kv,
-                   int max_seq, int S, hipStream_t s, int start_pos = 0) {
+                   int max_seq, int S, hipStream_t s, int start_pos = 0,
+                   _Float16 *out_planes = nullptr) {
   mia::FlashParams p{};
   int rt = 0;
   const int longest = positions == nullptr ? (int)std::min((long)start_pos + S, (long)max_seq) : max_seq;
   mia::flash_shared_plan(S, n_kv, kG, longest, c->num_cus, &p.n_rtiles, &p.nsplit, &rt);
   p.start_pos = start_pos;
+  p.S = S;
+  p.n_kv = n_kv;
+  set_out_planes(p, out_planes);
   p.Q = Q;
   p.rope_cs = rope_cs;
   p.positions = positions;
   p.kc = reinterpret_cast<const _Float16 *>(k_layer);
   p.vc = reinterpret_cast<const _Float16 *>(v_layer);
   p.out = out;
-  p.S = S;
-  p.n_kv = n_kv;
   p.max_seq = max_seq;
   p.qscale = qscale_log2();
   if (p.nsplit > 1) {
@@ -565,19 +573,25 @@ int check_positions(const int *positions, int S) {
   return MIA_OK;
 }
 
+// out_planes (not null): the output goes there as the next GEMM's fp16 hi and lo
+// planes [2][S][n_heads * 128] instead of to out.
 // With commit, the staged drafts kst/vst are copied into the ring after the
 // attention: by the split merge kernel when there is one, else by a copy
 // kernel.
 int flash_impl(DevCtx *c, const float *Q, const float *rope_cs, const uint16_t *kst,
                const uint16_t *vst, const uint16_t *k_layer, const uint16_t *v_layer, float *out,
-               int n_kv, int max_seq, int start_pos, int S, hipStream_t s, bool commit = false) {
+               int n_kv, int max_seq, int start_pos, int S, hipStream_t s, bool commit = false,
+               _Float16 *out_planes = nullptr) {
   const long keys = std::min((long)start_pos + S, (long)max_seq);
   if (kst == nullptr && S > kChunkFew && (long)n_kv * ((S + 7) / 8) <= c->num_cus &&
       (S > kShortOnly || keys <= kShortKeys))
     return positions_impl(c, Q, rope_cs, nullptr, k_layer, v_layer, out, n_kv, max_seq, S, s,
-                          start_pos);
+                          start_pos, out_planes);
   mia::FlashParams p{};
   int rt = 0;
+  p.S = S;
+  p.n_kv = n_kv;
+  set_out_planes(p, out_planes);
   mia::flash_plan(S, n_kv, kG, start_pos, max_seq, kst != nullptr, c->num_cus, &p.n_rtiles,
                   &p.nsplit, &p.split_keys, &rt);
   p.Q = Q;
@@ -587,8 +601,6 @@ int flash_impl(DevCtx *c, const float *Q, const float *rope_cs, const uint16_t *
   p.kstage = reinterpret_cast<const _Float16 *>(kst);
   p.vstage = reinterpret_cast<const _Float16 *>(vst);
   p.out = out;
-  p.S = S;
-  p.n_kv = n_kv;
   p.max_seq = max_seq;
   p.start_pos = start_pos;
   p.qscale = qscale_log2();
@@ -1338,7 +1350,8 @@ static int layer_run(DevCtx *c, float *X, const void *const (&ws)[7], const int 
   const int kv_dim = n_kv_heads * kHD;
   // gate and up in one launch, ending in the SwiGLU product
   const bool fused_ffn = types[4] == types[6] && !gemm_two_planes(types[4]);
-  // Q [S][dim] | K, V [S][kv_dim] | A [S][dim] | H planes [2][S][hidden] fp16,
+  // Q [S][dim] | K, V [S][kv_dim] | A planes [2][S][dim] fp16 (the attention's
+  // output as Wo's input) | H planes [2][S][hidden] fp16,
   // or, without the fused launch, G and U [S][hidden]; the normalised rows
   // (the QKV and W1 / W3 inputs) only exist as the GEMM's hi + lo planes in
   // split_work, written there by the RMSNorm, and the SwiGLU output H (W2's
@@ -1351,7 +1364,7 @@ static int layer_run(DevCtx *c, float *X, const void *const (&ws)[7], const int 
   float *Q = reinterpret_cast<float *>(w);
   float *K = reinterpret_cast<float *>(w + bd);
   float *V = reinterpret_cast<float *>(w + bd + bk);
-  float *A = reinterpret_cast<float *>(w + bd + 2 * bk);
+  _Float16 *const a_planes = reinterpret_cast<_Float16 *>(w + bd + 2 * bk);
   float *G = reinterpret_cast<float *>(w + 2 * bd + 2 * bk);
   float *U = reinterpret_cast<float *>(w + 2 * bd + 2 * bk + bh);
   _Float16 *const h_planes = reinterpret_cast<_Float16 *>(G);
@@ -1385,12 +1398,12 @@ static int layer_run(DevCtx *c, float *X, const void *const (&ws)[7], const int 
   HIP_TRY(mia::launch_rope_to_ring(K, V, theta_inv, S, start_pos, n_kv_heads,
                                    reinterpret_cast<_Float16 *>(k_layer),
                                    reinterpret_cast<_Float16 *>(v_layer), max_seq, cs, s));
-  if (int rc = flash_impl(c, Q, cs, nullptr, nullptr, k_layer, v_layer, A, n_kv_heads, max_seq,
-                          start_pos, S, s))
+  if (int rc = flash_impl(c, Q, cs, nullptr, nullptr, k_layer, v_layer, nullptr, n_kv_heads,
+                          max_seq, start_pos, S, s, false, a_planes))
     return rc;
   // X + A . Wo^T (vDSP_vadd after the GEMM: the sum rounded once more)
-  if (int rc = gemm_impl(c, types[3], ws[3], nullptr, nullptr, dim, 0, 0, A, dim, S, X, nullptr,
-                         nullptr, mia::kGemmAdd, s, packed))
+  if (int rc = gemm_impl(c, types[3], ws[3], nullptr, nullptr, dim, 0, 0, nullptr, dim, S, X,
+                         nullptr, nullptr, mia::kGemmAdd, s, packed, false, a_planes))
     return rc;
   HIP_TRY(mia::launch_rmsnorm_split(xn_hi, xn_lo, X, rms_ffn, dim, S, eps, s));
   if (fused_ffn) {

@@ -342,6 +342,32 @@ __device__ __forceinline__ void pv_drain_all(f16v (&o)[NB][4]) {
 __device__ __forceinline__ float half_swap_max(float m) { return fmaxf(m, __shfl_xor(m, 32)); }
 __device__ __forceinline__ float half_swap_sum(float x) { return x + __shfl_xor(x, 32); }
 
+// Output elements i .. i + 3 (of [S][n_heads * 128]): fp32, or, for the GEMM
+// that follows in a layer, its fp16 hi + lo planes (launch_split_hilo's split).
+__device__ __forceinline__ void store_out4(const FlashParams &p, size_t i, const f4 &v) {
+  if (p.out_hi == nullptr) {
+    *reinterpret_cast<f4 *>(p.out + i) = v;
+    return;
+  }
+  h4 hi, lo;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    hi[e] = (_Float16)v[e];
+    lo[e] = (_Float16)(v[e] - (float)hi[e]);
+  }
+  *reinterpret_cast<h4 *>(p.out_hi + i) = hi;
+  *reinterpret_cast<h4 *>(p.out_lo + i) = lo;
+}
+__device__ __forceinline__ void store_out(const FlashParams &p, size_t i, float v) {
+  if (p.out_hi == nullptr) {
+    p.out[i] = v;
+    return;
+  }
+  const _Float16 hi = (_Float16)v;
+  p.out_hi[i] = hi;
+  p.out_lo[i] = (_Float16)(v - (float)hi);
+}
+
 // Position of query t of a POS launch.
 __device__ __forceinline__ int query_pos(const FlashParams &p, int t) {
   return p.positions != nullptr ? p.positions[t] : p.start_pos + t;
@@ -403,17 +429,15 @@ __device__ __forceinline__ void rows_alone(const FlashParams &p, int kvh, int ti
       o0 = o0 * a + w * (float)p.vc[off];
       o1 = o1 * a + w * (float)p.vc[off + 1];
     }
-    float *dst = p.out + at;
     if (n_splits == 1) {
       const float inv = l == 0.f ? 0.f : 1.0f / l;
-      o0 *= inv;
-      o1 *= inv;
+      store_out(p, at, o0 * inv);
+      store_out(p, at + 1, o1 * inv);
     } else {
       const size_t row = ((size_t)tile_id * p.nsplit + split) * (32 * NB) + rl;
-      dst = p.part_o + row * HD + 2 * lane;
       if (lane == 0) store_shared2(p.part_ml + row * 2, m, l);
+      store_shared2(p.part_o + row * HD + 2 * lane, o0, o1);
     }
-    store_shared2(dst, o0, o1);
   }
 }
 
@@ -493,8 +517,7 @@ __device__ __forceinline__ void merge_last_split(const FlashParams &p, char *sme
 #pragma unroll
   for (int j = 0; j < RT / 8; ++j) {
     const int row = row0 + r0 + 8 * j, t = row >> 2, g = row & 3;
-    if (t < p.S)
-      *reinterpret_cast<f4 *>(p.out + ((size_t)t * p.n_kv * 4 + kvh * 4 + g) * HD + dim) = acc[j];
+    if (t < p.S) store_out4(p, ((size_t)t * p.n_kv * 4 + kvh * 4 + g) * HD + dim, acc[j]);
   }
 }
 
@@ -1522,9 +1545,9 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
         // dims 32*db + 8*q + 4*half .. +4 (the accumulator's dim order)
         if (n_splits == 1) {
           const float inv = POS && Ls == 0.f ? 0.f : 1.0f / Ls;  // (no keys: zeros)
-          float *dst = p.out + (size_t)t * dim_model + (size_t)(kvh * 4 + g) * HD + 32 * db + 4 * half;
+          const size_t at = (size_t)t * dim_model + (size_t)(kvh * 4 + g) * HD + 32 * db + 4 * half;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) *reinterpret_cast<f4 *>(dst + 8 * q) = acc[q] * inv;
+          for (int q = 0; q < 4; ++q) store_out4(p, at + 8 * q, acc[q] * inv);
         } else {
           const size_t pidx = (tile_id * p.nsplit + split) * RT + rl;
           float *dst = p.part_o + pidx * HD + 32 * db + 4 * half;
@@ -1632,7 +1655,7 @@ __global__ void __launch_bounds__(256) flash_merge_kernel(FlashParams p, int rt)
 #pragma unroll
     for (int k = 0; k < 32; ++k) sum += red[k][tid];
     const float Ls = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-    p.out[(size_t)t * (kv_dim * 4) + (size_t)(kvh * 4 + g) * HD + tid] = sum / Ls;
+    store_out(p, (size_t)t * (kv_dim * 4) + (size_t)(kvh * 4 + g) * HD + tid, sum / Ls);
   }
 }
 

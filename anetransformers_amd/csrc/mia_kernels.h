@@ -61,6 +61,7 @@ struct FlashParams {
   const _Float16 *kstage;  // [S][kv_dim] staged new keys (nullptr: all keys in ring)
   const _Float16 *vstage;
   float *out;              // [S][n_heads*128]
+  _Float16 *out_hi, *out_lo;  // not null: the output as fp16 hi + lo planes instead
   float *part_o;           // split-K partials (nsplit > 1)
   float *part_ml;
   _Float16 *commit_k;      // nsplit > 1 with staged drafts: the merge kernel copies
