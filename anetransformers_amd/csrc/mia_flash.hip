@@ -32,9 +32,9 @@
 // The scores of tile i+1 are computed on MFMA while the exponentials of tile
 // i are formed.  Each row's softmax reference is its first tile's max,
 // subtracted inside the score MFMA by one extra k-step, and stays until a
-// tile holds a score more than 15 log2 units above it (P's hi part is fp16):
-// the wave then raises the reference of such rows and scales what they have
-// summed so far, once per new peak.
+// tile holds a score too far above it for P's fp16 hi part: the wave then raises
+// the reference of such rows and scales what they have summed so far, once per
+// new peak.
 //
 // Query t at position start+t attends the window [pos-L+1, pos], L =
 // min(pos+1, max_seq) (mistral_ane_prefill.h:220-241); positions >= start come
@@ -834,14 +834,20 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   // Softmax reference per row: the max of the row's scores in its first tile
   // (p <= 1 there), rounded to fp16 hi + lo and subtracted inside the score
   // MFMA by one extra k-step (a ones column in K against -m_ref in Q).  P's
-  // hi part is fp16, so a score may lie up to 16 above the reference: as long
-  // as none lies more than kRaise above it, the loop only compares each
-  // tile's scores with a per-row limit (raise_ref below does the rest), which
-  // sits in issue slots under the P.V MFMAs.  Model attention has such peaks
-  // (a few keys far above the first ones), and a second pass over the keys
-  // for rows that overflowed, the form before this one, ran 70.5 us instead
-  // of 38 at S 512 over 2048 keys with every 1024th key four times as large.
+  // hi part is fp16, so a score may lie up to 16 (log2 units) above the
+  // reference.  Model attention has keys further above it than that (a few
+  // peaks far above the first keys), and the row then takes a higher one:
+  //   NB = 1  raise_ref, on the next tile's scores, once one is more than
+  //           kRaise above its reference;
+  //   NB = 2  redo_tile, once the sum of a tile's exponentials, which the step
+  //           forms anyway, passes kSumLimit.  These steps are bound by their
+  //           instruction count: comparing every score instead (26 instructions
+  //           more a step) cost 5 to 10 % of the kernel on keys without peaks.
+  // Us a step of S tokens, plain keys and with every 1024th key four times as
+  // large: 512 after 1536 36.8 and 39.6 (a second pass over the keys for rows
+  // that overflowed: 37.1 and 69.0), 1999 after 6007 433 and 439 (434 and 648).
   constexpr float kRaise = 15.0f;
+  constexpr float kSumLimit = 32768.0f;
   f16v o[NB][4];
   float m_ref[NB], l_run[NB];
   f16v s_cur[NB];
@@ -946,7 +952,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
     return d;
   };
-  // Called when a (masked) tile's scores sc, shifted by the present
+  // NB = 1: called when a (masked) tile's scores sc, shifted by the present
   // references, may exceed a row's limit: rows that do get their max as the
   // new reference (a row without one yet, whatever its max), and everything
   // that carries the old one is scaled: the tile's scores, P of the tile
@@ -1165,7 +1171,84 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
       for (int b = 0; b < NB; ++b) mfma_pv2(o[b][db], va[db], pb[b][1], pb[b][3]);
   };
 
-  // NB = 2 (prefill): the same step as 34 slots of one score k-step (hi and
+  // step2's way past a peak.  P of tile it may not fit its fp16 hi parts in some
+  // row (its sum ls in a lane is above kSumLimit; a value overflows at twice
+  // that), or some row has no reference yet.  The tile's
+  // scores are formed again, from K rows read from memory (their LDS buffer
+  // holds tile it + 2 by now), every row with a score above its reference
+  // takes its max as the new one, P and ls are formed with it, and what
+  // carries the old one is scaled: the next tile's scores, the row sum and O.
+  unsigned long long unset = 0;  // lanes with keys whose row has no reference
+  auto redo_tile = [&](int it, f16v(&s_next)[NB], h8(&pl)[NB][4], float(&ls)[NB]) {
+    const int kb = kb0 + kStride * it;
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const _Float16 *kr;  // the lane's key row (those past the range repeat its last)
+    if constexpr (FAST) {
+      kr = kc + (size_t)min(fast_slot(it) + (ln & 31), ke - 1) * kv_dim;
+    } else {
+      const int kp = min(kb + (ln & 31), ke - 1);
+      kr = kst != nullptr && kp >= p.start_pos ? kst + (size_t)(kp - p.start_pos) * kv_dim
+                                               : kc + (size_t)(kp % p.max_seq) * kv_dim;
+    }
+    kr += kvh * HD + 8 * (ln >> 5);
+    bool none = false;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      f16v sc;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+#pragma unroll
+      for (int st = 0; st < 8; ++st) {
+        const h8 ka = *reinterpret_cast<const h8 *>(kr + 16 * st);
+        fence();
+        if (st == 0) mfma_qk_first(sc, ka, qb[b][0], ql[b][0]);
+        else mfma_qk(sc, ka, qb[b][st], ql[b][st]);
+      }
+      asm volatile("s_nop 7\n\ts_nop 7" : "+v"(sc));
+      mask_block(sc, b, kb, FAST ? min(fast_slot(it), kb) : kb);
+      const float m = block_max(sc);
+      const bool first = m_ref[b] == -INFINITY;
+      const float old = first ? 0.f : m_ref[b];
+      if (m > m_ref[b]) set_ref(b, m);
+      none = none || m_ref[b] == -INFINITY;
+      const float ref = m_ref[b] == -INFINITY ? 0.f : m_ref[b];
+      const float f = first ? 1.f : fast_exp2(old - ref);  // (nothing was summed without one)
+      ls[b] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) {
+        const float p0 = fast_exp2(sc[e] - ref), p1 = fast_exp2(sc[e + 1] - ref);
+        ls[b] += p0 + p1;
+        unsigned hi, lo;
+        split_pair(p0, p1, hi, lo);
+        u4 vh = __builtin_bit_cast(u4, pl[b][e >> 3]), vl = __builtin_bit_cast(u4, pl[b][2 + (e >> 3)]);
+        vh[(e & 7) >> 1] = hi;
+        vl[(e & 7) >> 1] = lo;
+        pl[b][e >> 3] = __builtin_bit_cast(h8, vh);
+        pl[b][2 + (e >> 3)] = __builtin_bit_cast(h8, vl);
+      }
+      l_run[b] *= f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s_next[b][i] += old - ref;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        // (pinned before and after: one vector at a time passes through the
+        // VGPRs; all eight at once would spill Q in the loop around this)
+        fence();
+        asm volatile("" : "+a"(o[b][db]));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[b][db][i] *= f;
+        asm volatile("" : "+a"(o[b][db]));
+      }
+      fence();
+    }
+    unset = __builtin_amdgcn_ballot_w64(none);
+    // the accumulators were just written by the VALU, which the inline
+    // assembly MFMAs do not wait for
+    pv_drain_all(o);
+  };
+
+  // NB = 2: the same step as 34 slots of one score k-step (hi and
   // lo q) or one P.V k-step (hi and lo P), i.e. two MFMAs, except the two
   // reference k-steps; each slot is followed by one exponential of tile it
   // (with its hi + lo split and row-sum work every second slot), so the
@@ -1194,9 +1277,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
       vlo[3] = read_va<0, 3>(vab);
     }
     fence();
-    float ls[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) ls[b] = l_run[b];
+    float ls[NB];  // the tile's part of the row sum
     u4 pw[NB][4];  // hi parts (keys 0-15, 16-31), then lo parts
     float ex[4];
     // Element k of exponential slice j: score e = 4 (j % 4) + k of row block
@@ -1207,7 +1288,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     auto E = [&](int j, int k) {
       const int b = j >> 2, e = 4 * (j & 3) + k;
       ex[k] = fast_exp2(s_in[b][e]);
-      ls[b] += ex[k];
+      ls[b] = e == 0 ? ex[k] : ls[b] + ex[k];
       if (k & 1) {
         unsigned hi, lo;
         split_pair(ex[k - 1], ex[k], hi, lo);
@@ -1233,16 +1314,6 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     };
     auto PVH = [&](int db, int b) {
       if (with_pv) mfma_pv2(o[b][db], vhi[db], p_in[b][1], p_in[b][3]);
-    };
-    // Slice j (0 .. 7) of the new scores' maxima: four scores of block j / 4.
-    float mx[NB];
-    auto M = [&](int j) {
-      if (!with_qk) return;
-      const int b = j >> 2, e = 4 * (j & 3);
-      if (e == 0) mx[b] = s_out[b][0];
-      mx[b] = max3(mx[b], s_out[b][e], s_out[b][e + 1]);
-      mx[b] = max3(mx[b], s_out[b][e + 2], s_out[b][e + 3]);
-      asm volatile("" ::"v"(mx[b]));
     };
     // slots 1-10: reference k-steps and k-steps 0-3; exponential slices 0-2
     REF(0); fence(); E(0, 0); fence();
@@ -1306,17 +1377,15 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     fence();
     // slots 27-34: P.V keys 16-31; V(it+1) goes into V(it-1)'s buffer once
     // every LDS read of the step is done
-    PVH(0, 0); fence(); E(6, 2); M(0); fence();
-    PVH(0, 1); fence(); E(6, 3); M(1); fence();
-    PVH(1, 0); keep(vhi[0]); fence(); E(7, 0); M(2); fence();
-    PVH(1, 1); fence(); E(7, 1); M(3); fence();
-    PVH(2, 0); keep(vhi[1]); fence(); E(7, 2); M(4); fence();
-    PVH(2, 1); fence(); E(7, 3); M(5); fence();
+    PVH(0, 0); fence(); E(6, 2); fence();
+    PVH(0, 1); fence(); E(6, 3); fence();
+    PVH(1, 0); keep(vhi[0]); fence(); E(7, 0); fence();
+    PVH(1, 1); fence(); E(7, 1); fence();
+    PVH(2, 0); keep(vhi[1]); fence(); E(7, 2); fence();
+    PVH(2, 1); fence(); E(7, 3); fence();
     PVH(3, 0);
     keep(vhi[2]);
     fence();
-    M(6);
-    M(7);
     if (it + 1 < g_count) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       MIA_LOAD_V_NEXT(it + 1, (it + 1) & 1);
@@ -1330,18 +1399,19 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
     if (with_pv) pv_drain_all(o);
     fence();
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      l_run[b] = ls[b];
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int h = 0; h < 4; ++h) p_out[b][h] = __builtin_bit_cast(h8, pw[b][h]);
-    }
     // Window mask of tile it+1, only where it crosses a window edge.
     if (with_qk) {
       const int kbn = kb0 + kStride * (it + 1);
       if (needs_mask(kbn)) mask_tile(s_out, kbn);
-      // (a wave's only tile is followed by a scoring of no tile)
-      if (it + 1 < g_count && any_above(mx)) raise_ref(s_out, p_out);
     }
+    const bool over = ls[0] > kSumLimit || ls[NB - 1] > kSumLimit;
+    if (__builtin_expect((__builtin_amdgcn_ballot_w64(over) | unset) != 0, 0))
+      redo_tile(it, s_out, p_out, ls);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) l_run[b] += ls[b];
   };
   // O += P.V of the wave's last tile (its V in vt[(g_count-1)&1]) from P.
   // The MFMAs are inline assembly, invisible to the compiler's hazard
@@ -1400,11 +1470,12 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
 #pragma unroll
   for (int b = 0; b < NB; ++b)
     if (!has_keys[b]) set_ref(b, 0.f);
+  unset = __builtin_amdgcn_ballot_w64(m_ref[0] == -INFINITY || m_ref[NB - 1] == -INFINITY);
 
   // Loads are issued in the order K0 K1 V0 | K2 V1 | K3 V2 | ... (step it
   // issues K(it+2), then V(it+1)).  Step it needs K(it+1) and V(it-1): only
   // V(it), the last load issued, may still be pending.
-  if constexpr (NB == 2 && FAST) {
+  if constexpr (NB == 2) {
     // Step it exponentiates tile it and scores tile it+1; the last step
     // (it = g_count - 1) scores nothing.
     using T = std::true_type;

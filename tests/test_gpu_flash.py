@@ -253,6 +253,9 @@ def test_verify_step_65536_peaked_large_v():
     (4096, 500, 8, (64, 507)),           # 32-row tiles
     (300, 1000, 40, (5, 250)),           # wrapped windows (slots): rows that start mid-tile
     (300, 1000, 8, (5, 104, 250)),
+    (4096, 1500, 300, (131, 160, 1000, 1799)),  # 64-row tiles, split by wave: second tile to the last
+    (4096, 0, 270, (100, 128, 129, 269)),       # rows whose waves have one tile, or none
+    (2048, 2500, 320, (1, 1000, 2047)),         # a wrapped ring
 ])
 def test_attention_batch_peaks_raise_the_reference(M, start, S, peaks):
     # A few keys 16 times as large: scores reach +-70 log2 units, so rows
@@ -321,3 +324,29 @@ def test_attention_batch_tiles_and_splits(M, start, S):
             n = min(start + t + 1, M)
             exact = D.gqa_decode_f64(Q[t], kc[:n], vc[:n], 32, 8, 128, n, n - 1)
             D.check_close(out[t], exact, what=f"turn={turn} M={M} start={start} S={S} t={t}")
+
+
+@pytest.mark.parametrize("M,start,S,peaks", [
+    (600, 580, 40, (300, 577)),            # 64-row tiles with staged rows: the window's middle and end
+    (600, 1500, 33, (1000, 1200, 1499)),   # a wrapped window, split over workgroups or whole
+    (300, 2000, 70, (1800, 1999)),
+])
+def test_attention_step_peaks_next_to_staged_rows(M, start, S, peaks):
+    # The reference-raising path with per-lane key addresses (ring and staging
+    # buffer): a chunk that does not fit the ring beside its window, a few of
+    # the cached keys and one new key 16 times as large.
+    G.say(f"attention_step peaks M={M} start={start} S={S} at {peaks}")
+    g = D.rng(500 + S + M)
+    kc, vc = _peaked_large_v(g, M, M, sigma=1.0)
+    for p in peaks:
+        kc[p % M] = D.to_f16_bits(16.0 * D.f16_bits_to_f32(kc[p % M]))
+    Q, K, V = D.normal(g, (S, 4096)), D.normal(g, (S, 1024)), D.normal(g, (S, 1024))
+    K[S // 2] *= 16.0
+    # kn, vn: the rings as the library left them, whose new fp16 rows the queries attended
+    out, kn, vn = G.attention_step(kc, vc, Q, K, V, TH, M, start, S)
+    exact = np.empty((S, 4096))
+    for t in range(S):
+        kc[(start + t) % M], vc[(start + t) % M] = kn[(start + t) % M], vn[(start + t) % M]
+        q = D.rope_f64(Q[t], start + t, TH, 32, 128)
+        exact[t] = D.gqa_decode_f64(q, kc, vc, 32, 8, 128, M, start + t)
+    D.check_close(out, exact, what=f"step peaks M={M} start={start} S={S}")
