@@ -51,6 +51,7 @@
 
 #include "mia_device.h"
 #include "mia_kernels.h"
+#include "mia_window.h"
 
 namespace mia {
 
@@ -381,7 +382,7 @@ __device__ __forceinline__ int wave_max_int(int v) {
 }
 
 // Partial results that another workgroup of the same launch reads: stores past
-// this XCD's L2 and loads past it (device scope, 8 bytes each).  A release
+// this XCD's L2 and loads past it (device scope).  A release
 // fence instead writes the whole L2 back, once per wave: S 32 after 4064 keys
 // took 48 us with fences, 23 with these.
 typedef unsigned long long u64;
@@ -389,55 +390,74 @@ __device__ __forceinline__ void store_shared2(float *p, float a, float b) {
   __hip_atomic_store(reinterpret_cast<u64 *>(p), __builtin_bit_cast(u64, (f2){a, b}),
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void store_shared(float *p, float a) {
+  __hip_atomic_store(p, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ f2 load_shared2(const float *p) {
   return __builtin_bit_cast(f2, __hip_atomic_load(reinterpret_cast<const u64 *>(p), __ATOMIC_RELAXED,
                                                   __HIP_MEMORY_SCOPE_AGENT));
 }
 
-// The rows of a POS workgroup one by one in fp32, over the keys of each row
-// alone: a wave per row, two dims per lane.  In the tile loop a key past a
-// row's position has weight 0 in that row, which an infinite or NaN value there
-// turns into NaN; a workgroup with such a result comes here, so that a row
-// depends on its own window only.
+// Where a POS workgroup has a result that is not finite.  In the tile loop a key
+// past a row's position has weight 0 in that row, which an infinite or NaN value
+// there turns into NaN: rows that such a key spoilt are computed again, a token
+// at a time over its own keys only, so that a row depends on its own window
+// only.  Only keys past a token's position, up to ke, can have done that, so
+// those are searched first; a value inside every window that reaches it is the
+// rows' own and nothing is done.  Bounds: the search reads what the tiles did
+// (16 keys at a time); a token alone, 64 keys at a time, about 1 us per 64 keys.
 template <int NB>
-__device__ __forceinline__ void rows_alone(const FlashParams &p, int kvh, int tile_id, int row0,
-                                           int split, int n_splits, int ks, int ke) {
-  const int lane = threadIdx.x & 63;
+__device__ __forceinline__ void tokens_alone(const FlashParams &p, char *smem, int kvh, int tile_id,
+                                             int row0, int split, int n_splits, int ks, int ke) {
+  const int tid = threadIdx.x;
   const size_t kv_dim = (size_t)p.n_kv * HD;
-  for (int rl = threadIdx.x >> 6; rl < 32 * NB; rl += kWaves) {
-    const int t = (row0 + rl) >> 2, g = (row0 + rl) & 3;
-    if (t >= p.S) continue;
-    const size_t at = ((size_t)t * p.n_kv * 4 + kvh * 4 + g) * HD + 2 * lane;
-    const float2 q = *reinterpret_cast<const float2 *>(p.Q + at);
-    float q0 = q.x, q1 = q.y;
-    if (p.rope_cs != nullptr) {
-      const float2 cs = *reinterpret_cast<const float2 *>(p.rope_cs + (size_t)t * HD + 2 * lane);
-      rope_pair(q0, q1, cs.x, cs.y);
-    }
-    q0 *= p.qscale;
-    q1 *= p.qscale;
-    float m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
-    const int end = min(min(query_pos(p, t), p.max_seq - 1), ke - 1);
-    for (int k = ks; k <= end; ++k) {
-      const size_t off = (size_t)k * kv_dim + kvh * HD + 2 * lane;
-      const float s = wave_sum(q0 * (float)p.kc[off] + q1 * (float)p.kc[off + 1]);
-      const float mn = fmaxf(m, s);
-      const float a = m == -INFINITY ? 0.f : fast_exp2(m - mn);
-      const float w = s == -INFINITY ? 0.f : fast_exp2(s - mn);
-      m = mn;
-      l = l * a + w;
-      o0 = o0 * a + w * (float)p.vc[off];
-      o1 = o1 * a + w * (float)p.vc[off + 1];
-    }
-    if (n_splits == 1) {
-      const float inv = l == 0.f ? 0.f : 1.0f / l;
-      store_out(p, at, o0 * inv);
-      store_out(p, at + 1, o1 * inv);
-    } else {
-      const size_t row = ((size_t)tile_id * p.nsplit + split) * (32 * NB) + rl;
-      if (lane == 0) store_shared2(p.part_ml + row * 2, m, l);
-      store_shared2(p.part_o + row * HD + 2 * lane, o0, o1);
-    }
+  const int t0 = row0 >> 2, t1 = min(t0 + 8 * NB, p.S);
+  auto last_key = [&](int t) { return min(min(query_pos(p, t), p.max_seq - 1), ke - 1); };
+  int from = ke;
+  for (int t = t0; t < t1; ++t) from = min(from, last_key(t) + 1);
+  from = max(from, ks);
+  // the last key of from .. ke - 1 with a value that is not finite
+  int bad = -1;
+  for (int k = from + (tid >> 4); k < ke; k += 16) {
+    const h8 v = *reinterpret_cast<const h8 *>(p.vc + (size_t)k * kv_dim + kvh * HD + 8 * (tid & 15));
+    float f = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f = __builtin_fmaf((float)v[e], 0.f, f);
+    if (f != 0.f) bad = k;
+  }
+  bad = wave_max_int(bad);
+  int *const wave_bad = reinterpret_cast<int *>(smem);  // (LDS is free: a barrier came before)
+  if ((tid & 63) == 0) wave_bad[tid >> 6] = bad;
+  wait_vmcnt<0>();  // this wave's results have arrived: other waves replace some below
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kWaves; ++k) bad = max(bad, wave_bad[k]);
+  bad = __builtin_amdgcn_readfirstlane(bad);
+  if (bad < 0) return;  // whole workgroup
+  DecodeParams dp{};
+  dp.kc = const_cast<_Float16 *>(p.kc);
+  dp.vc = const_cast<_Float16 *>(p.vc);
+  dp.max_seq = p.max_seq;
+  dp.n_kv = p.n_kv;
+  dp.nchunk = 1;
+  dp.qscale = p.qscale;
+  for (int t = t0; t < t1; ++t) {
+    const int last = __builtin_amdgcn_readfirstlane(last_key(t));
+    if (last >= bad) continue;  // whole workgroup
+    __syncthreads();  // (LDS: the token before, or the search)
+    const size_t row = (size_t)t * p.n_kv * 4;
+    window::attend<window::kTable, kWaves, 1>(
+        dp, *reinterpret_cast<window::Smem<kWaves> *>(smem), 0, max(last + 1 - ks, 0), ks,
+        p.Q + row * HD, p.rope_cs == nullptr ? nullptr : p.rope_cs + (size_t)t * HD, kvh, 0,
+        [&](int g, int d, float M, float L, float O) {
+          if (n_splits == 1) {
+            store_out(p, (row + kvh * 4 + g) * HD + d, L > 0.f ? O / L : 0.f);
+          } else {
+            const size_t pr = ((size_t)tile_id * p.nsplit + split) * (32 * NB) + 4 * (t - t0) + g;
+            store_shared(p.part_o + pr * HD + d, O);
+            if (d == 0) store_shared2(p.part_ml + pr * 2, M, L);
+          }
+        });
   }
 }
 
@@ -1641,7 +1661,7 @@ __global__ void __launch_bounds__(256) flash_kernel(FlashParams p) {
   }
   if constexpr (POS) {
     if (__syncthreads_or(finite != 0.f))
-      rows_alone<NB>(p, kvh, (int)tile_id, row0, split, n_splits, ks, ke);
+      tokens_alone<NB>(p, smem, kvh, (int)tile_id, row0, split, n_splits, ks, ke);
     if (n_splits > 1) merge_last_split<NB>(p, smem, (int)tile_id, row0, n_splits);
   }
 }

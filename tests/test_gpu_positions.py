@@ -229,3 +229,83 @@ def test_attention_positions_rows_depend_on_their_own_window_only(M):
     for t in (0, 1, 3, 4, 5, 6, 7, 8, 9):
         ref = D.gqa_decode_f64(Q[t], kc[:M // 2], vc[:M // 2], 32, 8, 128, M // 2, int(positions[t]))
         D.check_close(out[t], ref, what=f"t={t}")
+
+
+@pytest.mark.parametrize("M,start,S,bad", [
+    (4096, 1000, 20, (1015,)),         # one range of keys, the value past 15 tokens
+    (8192, 6000, 20, (6003, 6015)),    # the keys split over workgroups
+    (4096, 1000, 300, (1140, 1290)),   # 16-token tiles with positions on the device
+])
+def test_rows_next_to_later_infinities(M, start, S, bad):
+    # Tokens at consecutive positions through mia_attention_positions: an
+    # infinite value at one token's key leaves the tokens before it as they are.
+    G.say(f"attention_positions M={M} start={start} S={S} infinities at {bad}")
+    lib = G.lib()
+    g = D.rng(850 + M + S)
+    kc, vc = D.ring(g, M, filled=start + S)
+    for k in bad:
+        vc[k, ::3] = 0x7C00
+    positions = np.arange(start, start + S, dtype=np.int32)
+    positions[S // 2:] = positions[S // 2:][::-1].copy()  # (not in order)
+    Q = D.normal(g, (S, 4096))
+    dkc, dvc, dq, dp = DB.from_array(kc), DB.from_array(vc), DB.from_array(Q), DB.from_array(positions)
+    dout = DB(S * 4096 * 4)
+    check(lib.mia_attention_positions(dq.ptr, dout.ptr, dkc.ptr, dvc.ptr, dp.ptr, 32, 8, 128, M,
+                                      S, None), "attention_positions")
+    check(lib.mia_stream_sync(None), "sync")
+    out = dout.download((S, 4096), np.float32)
+    for t in range(S):
+        pos = int(positions[t])
+        if pos >= min(bad):
+            assert not np.all(np.isfinite(out[t]))
+        elif S < 50 or t % 16 < 2:
+            ref = D.gqa_decode_f64(Q[t], kc, vc, 32, 8, 128, M, pos)
+            D.check_close(out[t], ref, what=f"t={t} pos={pos}")
+
+
+def _call_ms(fn, n=5):
+    lib = G.lib()
+    e0, e1 = ctypes.c_void_p(), ctypes.c_void_p()
+    check(lib.mia_event_create(ctypes.byref(e0)), "event")
+    check(lib.mia_event_create(ctypes.byref(e1)), "event")
+    fn()
+    check(lib.mia_event_record(e0, None), "record")
+    for _ in range(n):
+        fn()
+    check(lib.mia_event_record(e1, None), "record")
+    check(lib.mia_stream_sync(None), "sync")
+    ms = ctypes.c_float()
+    check(lib.mia_event_elapsed_ms(ctypes.byref(ms), e0, e1), "elapsed")
+    lib.mia_event_destroy(e0)
+    lib.mia_event_destroy(e1)
+    return ms.value / n
+
+
+@pytest.mark.parametrize("where,factor", [("inside", 2.0), ("past", 40.0)])
+def test_infinities_cost_a_bounded_time(where, factor):
+    # A value that is not finite inside every window is the rows' own: only the
+    # search for another cause comes on top.  One past some rows' windows has
+    # those tokens computed alone, a few times the work of the call at 64K keys.
+    # (A row at a time, key by key, took hundreds of times as long.)
+    G.say(f"attention_positions 64K ring, infinity {where}")
+    lib = G.lib()
+    M, S = 65536, 16
+    g = D.rng(860)
+    kc, vc = D.ring(g, M)
+    positions = np.arange(M - S, M, dtype=np.int32)
+    Q = D.normal(g, (S, 4096))
+    dkc, dvc, dq, dp = DB.from_array(kc), DB.from_array(vc), DB.from_array(Q), DB.from_array(positions)
+    dout = DB(S * 4096 * 4)
+
+    def call():
+        check(lib.mia_attention_positions(dq.ptr, dout.ptr, dkc.ptr, dvc.ptr, dp.ptr, 32, 8, 128, M,
+                                          S, None), "attention_positions")
+
+    clean = _call_ms(call)
+    for k in range(100, M - S, 4096) if where == "inside" else (M - 1,):
+        vc[k] = 0x7C00
+    dvc2 = DB.from_array(vc)
+    dvc = dvc2
+    bad = _call_ms(call)
+    print(f"clean {clean * 1e3:.1f} us, with infinities {where} {bad * 1e3:.1f} us", flush=True)
+    assert bad < factor * clean + 0.02
