@@ -781,12 +781,13 @@ __global__ __launch_bounds__(kGThreads, (GemmLay<SRC, TM>::kPerCU)) void gemm_ke
 }
 
 // Sum of the split partial products in split order, then the epilogue: one
-// thread per VEC consecutive columns of a token.
+// thread per VEC consecutive columns of a token, span workgroups per token
+// (in one grid dimension: the others end at 65,535).
 template <int MODE, int VEC>
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p) {
-  const int m = blockIdx.y;
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p, int span) {
+  const int m = blockIdx.x / span;
   const int cols = MODE == kGemmSwiGlu ? p.rows0 : p.N;
-  const int n = (blockIdx.x * 256 + threadIdx.x) * VEC;
+  const int n = ((int)(blockIdx.x % span) * 256 + threadIdx.x) * VEC;
   if (n >= cols) return;
   const size_t plane = (size_t)p.S * p.N;
   const float *src = p.part + (size_t)m * p.N + n;
@@ -893,12 +894,13 @@ hipError_t launch_mode(const GemmParams &p, hipStream_t s, hipEvent_t ev0, hipEv
   if (p.ksplit > 1) {
     const int cols = MODE == kGemmSwiGlu ? p.rows0 : p.N;
     // four columns per thread where every output row keeps 16-byte steps
-    if ((p.rows0 | p.rows01 | p.N) % 4 == 0)
-      hipLaunchKernelGGL((gemm_reduce_kernel<MODE, 4>), dim3((cols + 1023) / 1024, p.S), dim3(256),
-                         0, s, p);
+    const bool vec = (p.rows0 | p.rows01 | p.N) % 4 == 0;
+    const int span = vec ? (cols + 1023) / 1024 : (cols + 255) / 256;
+    const dim3 grid((unsigned)span * (unsigned)p.S);
+    if (vec)
+      hipLaunchKernelGGL((gemm_reduce_kernel<MODE, 4>), grid, dim3(256), 0, s, p, span);
     else
-      hipLaunchKernelGGL((gemm_reduce_kernel<MODE, 1>), dim3((cols + 255) / 256, p.S), dim3(256),
-                         0, s, p);
+      hipLaunchKernelGGL((gemm_reduce_kernel<MODE, 1>), grid, dim3(256), 0, s, p, span);
   }
   return hipGetLastError();
 }
