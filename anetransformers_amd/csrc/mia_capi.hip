@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <hipblaslt/hipblaslt.h>
 
+#include <atomic>
 #include <climits>
 #include <cstdarg>
 #include <cstdio>
@@ -67,6 +68,27 @@ struct LtPick {
   hipblasLtMatmulAlgo_t algo;
 };
 
+// Work of the row tiles that share keys (positions_impl) for one stream: the
+// splits' partials, counts per row tile, and the (cos, sin) table of a chunk of
+// up to kChunkScanMax tokens.  A stream keeps the area of its first such call
+// until mia_stream_destroy (for good if a captured call uses it), so calls on two
+// streams do not meet in one.  Streams beyond kWorkStreams, and
+// hipStreamPerThread, which is another stream in every thread, take the kernels
+// without an area (positions_few_impl, flash_plan's tiles).
+constexpr int kWorkStreams = 8;
+constexpr int kCountSets = 8;
+struct StreamWork {
+  hipStream_t stream = nullptr;  // null: free
+  float *part = nullptr;
+  // [kCountSets][num_cus], FlashParams::arrive: 0 between launches.  A launch
+  // counts in one set and clears the set of the third launch after it, so
+  // that counts which a race or a failed launch left reach no later call.
+  int *arrive = nullptr;
+  std::atomic<unsigned> launches{0};
+  float *cs = nullptr;
+  std::atomic<bool> captured{false};
+};
+
 struct DevCtx {
   bool ready = false;
   hipStream_t stream = nullptr;
@@ -86,8 +108,7 @@ struct DevCtx {
   size_t split_work_bytes = 0;
   int *owner = nullptr;  // long chunks of mia_attention_chunk: last token per ring slot, -1 at rest
   int owner_slots = 0;
-  int *arrive = nullptr;  // queries at positions of their own: splits done per row tile, 0 at rest
-  int arrive_tiles = 0;
+  StreamWork stream_work[kWorkStreams];
   // hipBLASLt: handle and workspace created on first use, the algorithm of
   // each shape picked on its first call (lt_gemm), operands and products
   hipblasLtHandle_t lt = nullptr;
@@ -110,7 +131,10 @@ struct DevCtx {
 
 DevCtx g_ctx[kMaxDevices];
 std::mutex g_mu;
+std::mutex g_work_mu;  // the owners in DevCtx::stream_work
 thread_local char g_err[512] = "";
+
+size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 int set_err(int code, const char *fmt, ...) {
   va_list ap;
@@ -184,17 +208,54 @@ int ensure_owner(DevCtx *c, int slots) {
   return MIA_OK;
 }
 
-int ensure_arrive(DevCtx *c, int tiles) {
-  if (tiles > c->arrive_tiles) {
-    HIP_TRY(hipDeviceSynchronize());
-    if (c->arrive) HIP_TRY(hipFree(c->arrive));
-    c->arrive = nullptr;
-    c->arrive_tiles = 0;
-    HIP_TRY(hipMalloc((void **)&c->arrive, (size_t)tiles * sizeof(int)));
-    HIP_TRY(hipMemset(c->arrive, 0, (size_t)tiles * sizeof(int)));
-    c->arrive_tiles = tiles;
+// The areas of DevCtx::stream_work, in one allocation (68 MB on 256 CUs).
+int alloc_stream_work(DevCtx *c) {
+  if (c->stream_work[0].part != nullptr) return MIA_OK;
+  const size_t part = mia::flash_shared_scratch(c->num_cus), counts = (size_t)kCountSets * c->num_cus * 4,
+               cs = (size_t)kChunkScanMax * kHD * sizeof(float), each = al256(part + counts + cs);
+  char *m = nullptr;
+  HIP_TRY(hipMalloc((void **)&m, each * kWorkStreams));
+  HIP_TRY(hipMemset(m, 0, each * kWorkStreams));
+  HIP_TRY(hipDeviceSynchronize());
+  for (StreamWork &w : c->stream_work) {
+    w.part = reinterpret_cast<float *>(m);
+    w.arrive = reinterpret_cast<int *>(m + part);
+    w.cs = reinterpret_cast<float *>(m + part + counts);
+    m += each;
   }
   return MIA_OK;
+}
+
+// The stream's area, or null if all have owners.
+StreamWork *stream_work(DevCtx *c, hipStream_t s) {
+  if (s == hipStreamPerThread) return nullptr;
+  std::lock_guard<std::mutex> lock(g_work_mu);
+  StreamWork *free = nullptr;
+  for (StreamWork &w : c->stream_work) {
+    if (w.stream == s) return &w;
+    if (w.stream == nullptr && free == nullptr) free = &w;
+  }
+  if (free != nullptr) free->stream = s;
+  return free;
+}
+
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st == hipStreamCaptureStatusActive;
+}
+
+// A captured call counts in the same set in every replay: the launch before its
+// row tiles clears all sets, the rotation (which takes this area, or null) where
+// there is one.
+int *captured_counts(DevCtx *c, hipStream_t s) {
+  StreamWork *w = capturing(s) ? stream_work(c, s) : nullptr;
+  if (w == nullptr) return nullptr;
+  w->captured = true;
+  return w->arrive;
 }
 
 int ensure_layer_work(DevCtx *c, size_t bytes) {
@@ -497,9 +558,10 @@ void set_out_planes(mia::FlashParams &p, _Float16 *planes) {
 }
 
 // S tokens at their own positions (device int32 [S]) over the ring as it
-// stands; rope_cs set: Q is raw and rotated in-kernel.
+// stands; rope_cs set: Q is raw and rotated in-kernel (and the launch before was
+// the rotation).  w: the stream's work area.
 // positions null: start_pos + t.  out_planes: flash_impl's.
-int positions_impl(DevCtx *c, const float *Q, const float *rope_cs, const int *positions,
+int positions_impl(DevCtx *c, StreamWork *w, const float *Q, const float *rope_cs, const int *positions,
                    const uint16_t *k_layer, const uint16_t *v_layer, float *out, int n_kv,
                    int max_seq, int S, hipStream_t s, int start_pos = 0,
                    _Float16 *out_planes = nullptr) {
@@ -521,12 +583,14 @@ int positions_impl(DevCtx *c, const float *Q, const float *rope_cs, const int *p
   p.qscale = qscale_log2();
   if (p.nsplit > 1) {
     const size_t ntile = (size_t)n_kv * p.n_rtiles;
-    if (int rc = ensure_scratch(c, mia::flash_scratch_bytes(n_kv, p.n_rtiles, p.nsplit, rt)))
-      return rc;
-    if (int rc = ensure_arrive(c, (int)ntile)) return rc;
-    p.part_o = reinterpret_cast<float *>(c->split);
+    p.part_o = w->part;
     p.part_ml = p.part_o + ntile * p.nsplit * rt * kHD;
-    p.arrive = c->arrive;
+    const unsigned n = w->launches.fetch_add(1);
+    p.arrive = w->arrive + (size_t)(n % kCountSets) * c->num_cus;
+    p.clear = w->arrive + (size_t)((n + 3) % kCountSets) * c->num_cus;
+    p.n_clear = c->num_cus;
+    if (rope_cs == nullptr && captured_counts(c, s) != nullptr)
+      HIP_TRY(mia::launch_clear_counts(w->arrive, kCountSets * c->num_cus, s));
   }
   hipEvent_t ev0, ev1;
   if (int rc = prof_pair(c, positions == nullptr ? 1 : 0, &ev0, &ev1)) return rc;
@@ -584,9 +648,12 @@ int flash_impl(DevCtx *c, const float *Q, const float *rope_cs, const uint16_t *
                _Float16 *out_planes = nullptr) {
   const long keys = std::min((long)start_pos + S, (long)max_seq);
   if (kst == nullptr && S > kChunkFew && (long)n_kv * ((S + 7) / 8) <= c->num_cus &&
-      (S > kShortOnly || keys <= kShortKeys))
-    return positions_impl(c, Q, rope_cs, nullptr, k_layer, v_layer, out, n_kv, max_seq, S, s,
-                          start_pos, out_planes);
+      (S > kShortOnly || keys <= kShortKeys)) {
+    StreamWork *w = stream_work(c, s);
+    if (w != nullptr)
+      return positions_impl(c, w, Q, rope_cs, nullptr, k_layer, v_layer, out, n_kv, max_seq, S, s,
+                            start_pos, out_planes);
+  }
   mia::FlashParams p{};
   int rt = 0;
   p.S = S;
@@ -666,8 +733,6 @@ int q4_impl(const void *Wq, const void *Wk, const void *Wv, const void *x_q8, co
 }
 
 }  // namespace
-
-static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // The GEMM's packed form of a matrix of a type other than Q4_0: the fp16 hi
 // plane [N][K], then for Q6_K / F32 the lo plane [N][K] and the row scales [N]
@@ -877,11 +942,11 @@ int mia_init(int device) {
   HIP_TRY(mia::prepare_gemm());
   HIP_TRY(hipGetSymbolAddress(&c.noalloc, HIP_SYMBOL(scratch)));
   HIP_TRY(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
-  // Scratch of mia_attention_chunk and mia_attention_positions up to
-  // kChunkScanMax tokens, so that their first call may be captured.
+  // The first call of mia_attention_chunk up to kChunkScanMax tokens and of
+  // mia_attention_positions may be captured.
+  if (int rc = alloc_stream_work(&c)) return rc;
   if (int rc = ensure_work(&c, (size_t)kChunkScanMax * kHD * sizeof(float))) return rc;
   if (int rc = ensure_scratch(&c, mia::flash_shared_scratch(c.num_cus))) return rc;
-  if (int rc = ensure_arrive(&c, c.num_cus)) return rc;
   c.ready = true;
   return MIA_OK;
 }
@@ -963,7 +1028,25 @@ int mia_stream_create(void **stream) {
 }
 
 int mia_stream_destroy(void *stream) {
-  if (stream) HIP_TRY(hipStreamDestroy(reinterpret_cast<hipStream_t>(stream)));
+  if (!stream) return MIA_OK;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  StreamWork *held = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_work_mu);
+    for (DevCtx &c : g_ctx)
+      for (StreamWork &w : c.stream_work)
+        if (w.stream == s && !w.captured) held = &w;
+  }
+  // (its area goes to another stream only once its work is done)
+  if (held != nullptr && hipStreamSynchronize(s) != hipSuccess) {
+    (void)hipGetLastError();
+    held = nullptr;
+  }
+  HIP_TRY(hipStreamDestroy(s));
+  if (held != nullptr) {
+    std::lock_guard<std::mutex> lock(g_work_mu);
+    held->stream = nullptr;
+  }
   return MIA_OK;
 }
 
@@ -1155,10 +1238,11 @@ int mia_attention_positions(const float *Q, float *out, const uint16_t *k_layer,
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
   hipStream_t s = pick_stream(c, stream);
-  if (S <= kChunkFew)
+  StreamWork *w = S <= kChunkFew ? nullptr : stream_work(c, s);
+  if (w == nullptr)
     return positions_few_impl(c, Q, nullptr, positions, k_layer, v_layer, out, n_kv_heads, max_seq,
                               S, s);
-  return positions_impl(c, Q, nullptr, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S, s);
+  return positions_impl(c, w, Q, nullptr, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S, s);
 }
 
 int mia_attention_chunk(const float *Q, const float *K, const float *V, const int *positions,
@@ -1182,18 +1266,25 @@ int mia_attention_chunk(const float *Q, const float *K, const float *V, const in
     if (int rc = ensure_owner(c, max_seq)) return rc;
     owner = c->owner;
   }
-  // (the rotation also leaves the (cos, sin) table from which the flash kernel
-  // rotates Q)
-  if (int rc = ensure_work(c, (size_t)S * kHD * sizeof(float))) return rc;
-  float *cs = reinterpret_cast<float *>(c->work);
+  // (for the flash kernel the rotation also leaves the (cos, sin) table from
+  // which it rotates Q)
+  StreamWork *w = S <= kChunkFew ? nullptr : stream_work(c, s);
+  float *cs = nullptr;
+  if (w != nullptr) {
+    cs = w->cs;
+    if (S > kChunkScanMax) {
+      if (int rc = ensure_work(c, (size_t)S * kHD * sizeof(float))) return rc;
+      cs = reinterpret_cast<float *>(c->work);
+    }
+  }
   HIP_TRY(mia::launch_rope_kv_positions(K, V, theta_inv, positions, S, n_kv_heads,
                                         reinterpret_cast<_Float16 *>(k_layer),
                                         reinterpret_cast<_Float16 *>(v_layer), max_seq, owner,
-                                        cs, s));
-  if (S <= kChunkFew)
+                                        cs, captured_counts(c, s), kCountSets * c->num_cus, s));
+  if (w == nullptr)
     return positions_few_impl(c, Q, theta_inv, positions, k_layer, v_layer, out, n_kv_heads,
                               max_seq, S, s);
-  return positions_impl(c, Q, cs, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S, s);
+  return positions_impl(c, w, Q, cs, positions, k_layer, v_layer, out, n_kv_heads, max_seq, S, s);
 }
 
 int mia_attention_step(const float *Q, const float *K, const float *V, const float *theta_inv,
@@ -1226,7 +1317,8 @@ int mia_attention_step(const float *Q, const float *K, const float *V, const flo
   if (direct) {
     HIP_TRY(mia::launch_rope_to_ring(K, V, theta_inv, S, start_pos, n_kv_heads,
                                      reinterpret_cast<_Float16 *>(k_layer),
-                                     reinterpret_cast<_Float16 *>(v_layer), max_seq, cs, s));
+                                     reinterpret_cast<_Float16 *>(v_layer), max_seq, cs,
+                                     captured_counts(c, s), kCountSets * c->num_cus, s));
     return flash_impl(c, Q, cs, nullptr, nullptr, k_layer, v_layer, out, n_kv_heads, max_seq,
                       start_pos, S, s);
   }
@@ -1397,7 +1489,8 @@ static int layer_run(DevCtx *c, float *X, const void *const (&ws)[7], const int 
   float *cs = reinterpret_cast<float *>(c->work);
   HIP_TRY(mia::launch_rope_to_ring(K, V, theta_inv, S, start_pos, n_kv_heads,
                                    reinterpret_cast<_Float16 *>(k_layer),
-                                   reinterpret_cast<_Float16 *>(v_layer), max_seq, cs, s));
+                                   reinterpret_cast<_Float16 *>(v_layer), max_seq, cs,
+                                   captured_counts(c, s), kCountSets * c->num_cus, s));
   if (int rc = flash_impl(c, Q, cs, nullptr, nullptr, k_layer, v_layer, nullptr, n_kv_heads,
                           max_seq, start_pos, S, s, false, a_planes))
     return rc;

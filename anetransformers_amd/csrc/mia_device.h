@@ -57,6 +57,14 @@ __device__ __forceinline__ float wave_max(float x) {
   return x;
 }
 
+// Thread i of n_threads clears its part of n counts that another launch's
+// workgroups share (null: none).
+__device__ __forceinline__ void clear_counts(int *counts, int i, int n_threads, int n) {
+  if (counts == nullptr) return;
+  for (; i < n; i += n_threads)
+    __hip_atomic_store(counts + i, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Keeps the compiler from moving LDS accesses across this point; LDS

@@ -48,10 +48,11 @@ __global__ void rope_kernel(float *q, float *k, int S, int start_pos, const floa
 __global__ void __launch_bounds__(128)
     rope_kv_f16_kernel(const float *K, const float *V, const float *theta_inv, int S, int start_pos,
                        int n_kv, _Float16 *kdst, _Float16 *vdst, int max_seq, bool ring,
-                       float *cs_out) {
+                       float *cs_out, int *counts, int n_counts) {
   __shared__ float2 cs[HD / 2];
   const int t = blockIdx.x;
   const int tid = threadIdx.x;
+  clear_counts(counts, t * 128 + tid, S * 128, n_counts);
   const int pos = start_pos + t;
   const int kv_dim = n_kv * HD;
   const int n_items = n_kv * (HD / 8);
@@ -128,14 +129,16 @@ __global__ void slot_claim_kernel(const int *positions, int S, int max_seq, int 
 __global__ void __launch_bounds__(128)
     rope_kv_positions_kernel(const float *K, const float *V, const float *theta_inv,
                              const int *positions, int S, int n_kv, _Float16 *kc, _Float16 *vc,
-                             int max_seq, int *owner, float *cs_out) {
+                             int max_seq, int *owner, float *cs_out,
+                             int *counts, int n_counts) {
   __shared__ float2 cs[HD / 2];
   __shared__ int overwritten;
   const int t = blockIdx.x;
   const int tid = threadIdx.x;
+  clear_counts(counts, t * 128 + tid, S * 128, n_counts);
   const int pos = positions[t];
   if (pos < 0) {  // no slot (the attention gives such a token a zero row)
-    if (tid < HD / 2)
+    if (cs_out && tid < HD / 2)
       *reinterpret_cast<float2 *>(cs_out + (size_t)t * HD + 2 * tid) = make_float2(1.f, 0.f);
     return;
   }
@@ -174,7 +177,7 @@ __global__ void __launch_bounds__(128)
     float sn, c;
     sincosf(ang, &sn, &c);
     cs[tid] = make_float2(c, sn);
-    *reinterpret_cast<float2 *>(cs_out + (size_t)t * HD + 2 * tid) = cs[tid];
+    if (cs_out) *reinterpret_cast<float2 *>(cs_out + (size_t)t * HD + 2 * tid) = cs[tid];
   }
   __syncthreads();
   if (overwritten) return;  // workgroup-uniform
@@ -283,16 +286,17 @@ hipError_t launch_rope_to_f16(const float *K, const float *V, const float *theta
                               float *cs_out, hipStream_t s) {
   if (S <= 0) return hipSuccess;
   hipLaunchKernelGGL(rope_kv_f16_kernel, dim3(S), dim3(128), 0, s, K, V, theta_inv, S, start_pos,
-                     n_kv, kdst, vdst, 1, false, cs_out);
+                     n_kv, kdst, vdst, 1, false, cs_out, nullptr, 0);
   return hipGetLastError();
 }
 
 hipError_t launch_rope_to_ring(const float *K, const float *V, const float *theta_inv, int S,
                                int start_pos, int n_kv, _Float16 *kc, _Float16 *vc, int max_seq,
-                               float *cs_out, hipStream_t s) {
+                               float *cs_out, int *counts, int n_counts,
+                               hipStream_t s) {
   if (S <= 0) return hipSuccess;
   hipLaunchKernelGGL(rope_kv_f16_kernel, dim3(S), dim3(128), 0, s, K, V, theta_inv, S, start_pos,
-                     n_kv, kc, vc, max_seq, true, cs_out);
+                     n_kv, kc, vc, max_seq, true, cs_out, counts, n_counts);
   return hipGetLastError();
 }
 
@@ -308,7 +312,7 @@ hipError_t launch_kv_write(_Float16 *kc, _Float16 *vc, const float *K, const flo
 hipError_t launch_rope_kv_positions(const float *K, const float *V, const float *theta_inv,
                                     const int *positions, int S, int n_kv, _Float16 *kc,
                                     _Float16 *vc, int max_seq, int *owner, float *cs_out,
-                                    hipStream_t s) {
+                                    int *counts, int n_counts, hipStream_t s) {
   if (S <= 0) return hipSuccess;
   if (owner != nullptr) {
     hipLaunchKernelGGL(slot_claim_kernel, dim3((S + 255) / 256), dim3(256), 0, s, positions, S,
@@ -317,7 +321,7 @@ hipError_t launch_rope_kv_positions(const float *K, const float *V, const float 
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(rope_kv_positions_kernel, dim3(S), dim3(128), 0, s, K, V, theta_inv,
-                     positions, S, n_kv, kc, vc, max_seq, owner, cs_out);
+                     positions, S, n_kv, kc, vc, max_seq, owner, cs_out, counts, n_counts);
   return hipGetLastError();
 }
 

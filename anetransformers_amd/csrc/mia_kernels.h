@@ -72,7 +72,10 @@ struct FlashParams {
   int split_keys;          // keys per split (multiple of 64)
   float qscale;
   const int *positions;    // launch_flash_shared: the queries' positions [S], or null
-  int *arrive;             // and, with nsplit > 1, a count per row tile, 0 at rest
+  // and, with nsplit > 1, a count per row tile, 0 at rest, and n_clear counts of
+  // other launches to clear
+  int *arrive, *clear;
+  int n_clear;
 };
 size_t flash_scratch_bytes(int n_kv, int n_rtiles, int nsplit, int rows_per_tile);
 // Main kernel only; launch_flash_merge adds the split merge (nsplit > 1).
@@ -91,18 +94,21 @@ void flash_shared_plan(int S, int n_kv, int G, int longest, int target_wgs, int 
 size_t flash_shared_scratch(int target_wgs);
 hipError_t launch_flash_shared(const FlashParams &p, int G, hipStream_t s, hipEvent_t ev0,
                                hipEvent_t ev1);
+hipError_t launch_clear_counts(int *counts, int n, hipStream_t s);
 
 // Elementwise helpers.
 hipError_t launch_rope(float *q, float *k, int S, int start_pos, const float *theta_inv,
                        int n_heads, int n_kv, hipStream_t s);
 // K rotated and K, V rounded to fp16 into a dense staging buffer or the ring;
-// cs_out (may be null) receives the [S][64] (cos, sin) table of the positions.
+// cs_out (may be null) receives the [S][64] (cos, sin) table of the positions;
+// counts (may be null): n_counts counts to clear.
 hipError_t launch_rope_to_f16(const float *K, const float *V, const float *theta_inv, int S,
                               int start_pos, int n_kv, _Float16 *kdst, _Float16 *vdst,
                               float *cs_out, hipStream_t s);
 hipError_t launch_rope_to_ring(const float *K, const float *V, const float *theta_inv, int S,
                                int start_pos, int n_kv, _Float16 *kc, _Float16 *vc, int max_seq,
-                               float *cs_out, hipStream_t s);
+                               float *cs_out, int *counts, int n_counts,
+                               hipStream_t s);
 hipError_t launch_kv_write(_Float16 *kc, _Float16 *vc, const float *K, const float *V, int S,
                            int start_pos, int max_seq, int kv_dim, hipStream_t s);
 // The chunked prefill's phase 1 (mistral_model.h:935-955) for the K / V side:
@@ -111,11 +117,11 @@ hipError_t launch_kv_write(_Float16 *kc, _Float16 *vc, const float *K, const flo
 // chunk takes the same slot (the reference's in-order writes leave the last).
 // owner: null (each token scans the later ones, O(S^2) reads: short chunks)
 // or an int32 [max_seq] area holding -1 everywhere, left so (linear in S).
-// cs_out receives the [S][64] (cos, sin) table of the positions.
+// cs_out, counts: as launch_rope_to_ring's.
 hipError_t launch_rope_kv_positions(const float *K, const float *V, const float *theta_inv,
                                     const int *positions, int S, int n_kv, _Float16 *kc,
                                     _Float16 *vc, int max_seq, int *owner, float *cs_out,
-                                    hipStream_t s);
+                                    int *counts, int n_counts, hipStream_t s);
 // Staged rows 0..S-1 -> ring slots (start_pos + t) % max_seq, for n_layers
 // layers ring_stride / stage_stride elements apart.
 hipError_t launch_commit(_Float16 *kc, _Float16 *vc, const _Float16 *kst, const _Float16 *vst,

@@ -19,8 +19,14 @@
  *   - Calls that use device scratch (the split-K partials of the attention
  *     and GEMM kernels, the GEMM's fp16 hi / lo activation planes) share one
  *     per-device area of each kind: calls that overlap on one device
- *     (several host threads, or several streams) race.  The first call at a new size may allocate (not inside a HIP
- *     graph capture: warm up first).
+ *     (several host threads, or several streams) race, which spoils those
+ *     calls and no later ones.  mia_attention_positions and mia_attention_chunk of
+ *     9 tokens and more (of up to 64 in a chunk) use an area of their stream's
+ *     instead, so that such calls may overlap on different streams; a stream
+ *     holds one from its first such call to mia_stream_destroy, and calls on
+ *     more than 8 streams, or on hipStreamPerThread, take slower kernels.
+ *     The first call at a new size may allocate (not inside a HIP graph
+ *     capture: warm up first).
  */
 #ifndef MIATTN_H
 #define MIATTN_H
