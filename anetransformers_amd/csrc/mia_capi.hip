@@ -45,18 +45,25 @@ constexpr int kChunkScanMax = 64;
 //       32    9.8   11.5      15.7   17.7   37.2   22.0   64.9   26.2
 //       64   15.1   11.7      27.3   19.2   70.3   24.0  125.6   32.4
 constexpr int kChunkFew = 8;
-// Unstaged steps take the same kernel where its 32-row tiles fit the device at
-// once, except kChunkFew and fewer tokens, and up to kShortOnly tokens after
-// more than kShortKeys keys (separate merge: 20.6 us, here 22.0, 16 tokens
-// after 4064 keys).  Us a layer with 64-row tiles and the merge as a launch of
-// its own, then here:
-//   tokens   after 64 keys   700           2048          6000
-//       16   12.4    9.3     16.6   14.3   18.2   18.8   21.6   22.9
-//       64   12.8    9.8     24.3   14.4   27.4   20.5   32.2   28.3
-//      128   13.5   11.1     33.8   15.5   38.9   23.8   49.1   40.1
-//      256   15.6   12.5     51.9   17.4   60.1   28.6   86.5   63.9
-constexpr int kShortOnly = 16;
-constexpr int kShortKeys = 1024;
+// Unstaged steps of more than kChunkFew tokens take the same kernel where its
+// 32-row tiles fit the device at once and shared_tiles_pay: a tile is split into
+// eight ranges of keys at most, and 64-row tiles do less work per key, so the
+// keys up to which it is the faster one grow with the number of tiles.  Us a
+// step, 64-row tiles with the merge as a launch of its own, then here (tiles:
+// kv heads x tokens / 8):
+//   tiles   256 keys     800          1024         2048         4096         8192
+//       3   10.0   8.0   13.3  12.9   12.9  14.2   12.8  16.0   12.9  18.2   14.0  20.4
+//      16   10.4   8.0   14.0  12.5   13.7  13.4   14.5  14.6   17.7  18.2   18.0  21.7
+//      24   10.3   7.9   16.0  12.5   16.5  13.3   17.6  16.0   17.1  18.1   19.6  21.5
+//      32   10.2   8.2   16.1  12.4   16.8  13.4   19.1  17.5   19.8  18.8   21.3  23.6
+//      64   10.6   8.3   21.7  12.8   22.9  13.5   23.6  17.2   26.2  20.8   30.9  29.2
+//     128   10.8   8.6   30.7  12.9   31.0  14.0   33.7  19.9   39.9  28.3   51.5  45.8
+//     256   10.9   8.6   47.7  13.7   48.3  14.8   54.0  24.4   67.3  41.4   93.9  76.9
+// 128 tiles: 65.3 and 62.6 at 12,288 keys, 79.2 and 80.4 at 16,384, 250 and 300 at
+// 65,536; 3 tiles there: 21.0 and 78.0.
+bool shared_tiles_pay(long tiles, long keys) {
+  return keys <= 900 || (keys <= 12288 && keys <= (tiles < 20 ? 64 : 160) * tiles);
+}
 // The K and V projections of layers of other weight types (hipBLASLt): workspace
 // size, algorithms timed on a shape's first call, shapes remembered.
 constexpr size_t kLtWorkspace = size_t(64) << 20;
@@ -647,8 +654,8 @@ int flash_impl(DevCtx *c, const float *Q, const float *rope_cs, const uint16_t *
                int n_kv, int max_seq, int start_pos, int S, hipStream_t s, bool commit = false,
                _Float16 *out_planes = nullptr) {
   const long keys = std::min((long)start_pos + S, (long)max_seq);
-  if (kst == nullptr && S > kChunkFew && (long)n_kv * ((S + 7) / 8) <= c->num_cus &&
-      (S > kShortOnly || keys <= kShortKeys)) {
+  const long tiles = (long)n_kv * ((S + 7) / 8);
+  if (kst == nullptr && S > kChunkFew && tiles <= c->num_cus && shared_tiles_pay(tiles, keys)) {
     StreamWork *w = stream_work(c, s);
     if (w != nullptr)
       return positions_impl(c, w, Q, rope_cs, nullptr, k_layer, v_layer, out, n_kv, max_seq, S, s,

@@ -14,6 +14,7 @@ import _gpu as G
 import _oracle as O
 from anetransformers_amd import DeviceBuffer as DB
 from anetransformers_amd import check
+from test_gpu_positions import _call_ms
 from test_zz_no_alloc import _hip
 
 pytestmark = pytest.mark.gpu
@@ -25,8 +26,8 @@ M = 8192
 class Call:
     """One entry point on its own ring and inputs, rows at start .. start + S - 1 (n_kv kv heads)."""
 
-    def __init__(self, op, start, S, seed, n_kv=8):
-        self.op, self.start, self.S, self.n_kv = op, start, S, n_kv
+    def __init__(self, op, start, S, seed, n_kv=8, M=M):
+        self.op, self.start, self.S, self.n_kv, self.M = op, start, S, n_kv, M
         g = D.rng(seed)
         kv, dim = n_kv * 128, n_kv * 512
         self.kc, self.vc = D.ring(g, M, kv_dim=kv, filled=start)
@@ -44,15 +45,15 @@ class Call:
         lib, heads, S = G.lib(), 4 * self.n_kv, self.S
         if self.op == "positions":
             rc = lib.mia_attention_positions(Q, out.ptr, kc, vc, self.pos.ptr, heads, self.n_kv,
-                                             128, M, S, stream)
+                                             128, self.M, S, stream)
         elif self.op == "batch":
-            rc = lib.mia_attention_batch(Q, out.ptr, kc, vc, heads, self.n_kv, 128, M, self.start, S,
+            rc = lib.mia_attention_batch(Q, out.ptr, kc, vc, heads, self.n_kv, 128, self.M, self.start, S,
                                          stream)
         elif self.op == "chunk":
             rc = lib.mia_attention_chunk(Q, K, V, self.pos.ptr, th, kc, vc, out.ptr, heads,
-                                         self.n_kv, 128, M, S, stream)
+                                         self.n_kv, 128, self.M, S, stream)
         else:
-            rc = lib.mia_attention_step(Q, K, V, th, kc, vc, out.ptr, heads, self.n_kv, 128, M,
+            rc = lib.mia_attention_step(Q, K, V, th, kc, vc, out.ptr, heads, self.n_kv, 128, self.M,
                                         self.start, S, stream)
         check(rc, self.op)
 
@@ -186,3 +187,32 @@ def test_fewer_kv_heads(op, n_kv, S):
     for t in sorted({0, 1, 7, 8, S // 2, S - 2, S - 1}):
         exact = D.gqa_decode_f64(Q[t], kc, vc, 4 * n_kv, n_kv, 128, M, c.start + t)
         D.check_close(got[t], exact, what=f"{op} n_kv={n_kv} S={S} t={t}")
+
+
+@pytest.mark.parametrize("n_kv,S,M,keys", [
+    (1, 17, 4096, 900), (1, 17, 4096, 901),      # short windows: tiles that share keys at any count
+    (8, 16, 4096, 1024), (8, 16, 4096, 1025),    # 16 tiles
+    (8, 24, 4096, 3840), (8, 24, 4096, 3841),    # 24 tiles
+    (8, 80, 16384, 12288), (8, 80, 16384, 12289),
+])
+def test_batch_where_the_kernel_changes(n_kv, S, M, keys):
+    G.say(f"attention_batch n_kv={n_kv} S={S} keys={keys}")
+    c = Call("batch", keys - S, S, 80, n_kv, M)
+    got = c.alone()
+    for t in sorted({0, 7, 8, S - 2, S - 1}):
+        exact = D.gqa_decode_f64(c.Q[t], c.kc, c.vc, 4 * n_kv, n_kv, 128, M, c.start + t)
+        D.check_close(got[t], exact, what=f"n_kv={n_kv} S={S} keys={keys} t={t}")
+
+
+def test_long_windows_of_few_rows_use_the_device():
+    # 17 tokens of one kv head: three row tiles.  With eight ranges of keys a tile
+    # the step took 4.3 times as long after 64K keys as after 4K; split over the
+    # device it takes 1.6 times as long.
+    G.say("attention_batch n_kv=1 S=17, 4K and 64K keys")
+    ms = []
+    for keys in (4096, 65536):
+        c = Call("batch", keys - 17, 17, 81, 1, keys)
+        out = c.buffer()
+        ms.append(min(_call_ms(lambda: c(out, None), 20) for _ in range(3)))
+    print(f"{ms[0] * 1e3:.1f} us, {ms[1] * 1e3:.1f} us", flush=True)
+    assert ms[1] < 2.7 * ms[0]
