@@ -34,17 +34,31 @@ constexpr int kMaxSeq = 1 << 22;  // ring capacity limit; in-layer offsets are 6
 // token takes its slot by scanning them (S^2 / 2 reads); longer chunks use a
 // per-slot area instead (one more launch, linear in S).
 constexpr int kChunkScanMax = 64;
-// mia_attention_chunk, mia_attention_positions: up to this many tokens go
-// through the decode kernel, each reading its own window; more through the flash
-// kernel, whose row tiles share the keys among 8 tokens.  Us a layer, decode
-// then flash kernel (rotation of K included, 8 kv heads):
-//   tokens   after 256 keys   1024          4064          8000
-//        4   11.1   11.6      12.1   17.2   14.9   20.3   18.9   23.9
-//        8   12.5   11.4      13.8   17.6   19.8   20.5   27.2   23.7
-//       12   17.7   11.7      21.8   17.7   36.1   21.1   54.6   24.7
-//       32    9.8   11.5      15.7   17.7   37.2   22.0   64.9   26.2
-//       64   15.1   11.7      27.3   19.2   70.3   24.0  125.6   32.4
+// mia_attention_chunk, mia_attention_positions: few tokens go through the decode
+// kernel, each reading its own window; more through the flash kernel, whose row
+// tiles share the keys among 8 tokens.  The host knows the ring, not the windows.
+// Us of mia_attention_positions on a ring of 8192, decode kernel then flash kernel
+// (workgroups of the decode kernel before it splits the windows: tokens x kv
+// heads):
+//   kv heads, tokens   256 keys     512          1024         2048         8192
+//         1   9        10.2   8.0   11.2   9.9   11.2  14.1   11.7  16.1   14.5  20.5
+//         1  16         9.0   7.8    9.0   9.6    9.8  13.0    9.9  16.3   12.2  20.6
+//         1  32         9.7   7.9    9.4   9.7    9.7  13.3   11.1  15.8   16.5  20.2
+//         1  40        11.9   8.0   12.3   9.6   13.7  13.3   15.2  16.3   28.9  20.7
+//         2  16         8.5   8.0    9.4   9.6    9.7  13.3   11.3  15.9   16.5  20.2
+//         2  24        11.6   7.9   13.3   9.7   13.9  13.2   16.8  16.1   32.2  20.7
+//         8   9        12.5   8.3   13.5  10.0   15.3  14.4   19.6  15.9   42.3  21.7
+//         8  24        16.6   8.2   19.1   9.8   22.7  13.3   30.6  16.1   73.2  22.4
+//         8  32         6.5   8.0    8.4  10.0   12.5  13.3   20.4  16.2   66.1  23.8
+//         8  40        11.1   8.0   14.9   9.8   22.7  13.3   37.1  16.3  121.7  25.6
+// Where each token of each head is one workgroup and they fill the device (32
+// tokens of 8 heads) the decode kernel is the faster one up to 1,100 keys, and
+// taken where the ring is no longer than that.
 constexpr int kChunkFew = 8;
+bool few_positions(int S, int n_kv, int max_seq, int num_cus) {
+  const long wgs = (long)S * n_kv;
+  return S <= kChunkFew || wgs <= 32 || (wgs == num_cus && max_seq <= 1024);
+}
 // Unstaged steps of more than kChunkFew tokens take the same kernel where its
 // 32-row tiles fit the device at once and shared_tiles_pay: a tile is split into
 // eight ranges of keys at most, and 64-row tiles do less work per key, so the
@@ -1245,7 +1259,7 @@ int mia_attention_positions(const float *Q, float *out, const uint16_t *k_layer,
   DevCtx *c;
   if (int rc = current_ctx(&c)) return rc;
   hipStream_t s = pick_stream(c, stream);
-  StreamWork *w = S <= kChunkFew ? nullptr : stream_work(c, s);
+  StreamWork *w = few_positions(S, n_kv_heads, max_seq, c->num_cus) ? nullptr : stream_work(c, s);
   if (w == nullptr)
     return positions_few_impl(c, Q, nullptr, positions, k_layer, v_layer, out, n_kv_heads, max_seq,
                               S, s);
@@ -1275,7 +1289,7 @@ int mia_attention_chunk(const float *Q, const float *K, const float *V, const in
   }
   // (for the flash kernel the rotation also leaves the (cos, sin) table from
   // which it rotates Q)
-  StreamWork *w = S <= kChunkFew ? nullptr : stream_work(c, s);
+  StreamWork *w = few_positions(S, n_kv_heads, max_seq, c->num_cus) ? nullptr : stream_work(c, s);
   float *cs = nullptr;
   if (w != nullptr) {
     cs = w->cs;

@@ -150,8 +150,9 @@ int mia_attention_batch(const float *Q, float *out, const uint16_t *k_layer,
  * (mistral/mistral_model.h:961-1044), which is gqa_attention_neon per token.
  * Q [S][n_heads*128] fp32 dev, rotated; positions [S] int32 dev (any order,
  * >= 0; a negative position gives a zero row); out [S][n_heads*128].
- * 1 <= S <= 65535.  Above 8 tokens, 8 consecutive tokens (16 in long
- * batches) share one pass over the ring, up to their largest position. */
+ * 1 <= S <= 65535.  Above 8 tokens (32 / n_kv_heads on few kv heads), 8
+ * consecutive tokens (16 in long batches) share one pass over the ring, up to
+ * their largest position. */
 int mia_attention_positions(const float *Q, float *out, const uint16_t *k_layer,
                             const uint16_t *v_layer, const int *positions, int n_heads,
                             int n_kv_heads, int hd, int max_seq, int S, void *stream);

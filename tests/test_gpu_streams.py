@@ -216,3 +216,35 @@ def test_long_windows_of_few_rows_use_the_device():
         ms.append(min(_call_ms(lambda: c(out, None), 20) for _ in range(3)))
     print(f"{ms[0] * 1e3:.1f} us, {ms[1] * 1e3:.1f} us", flush=True)
     assert ms[1] < 2.7 * ms[0]
+
+
+@pytest.mark.parametrize("n_kv,S,M,keys", [
+    (1, 32, 4096, 3000), (1, 33, 4096, 3000), (2, 16, 4096, 3000), (2, 17, 4096, 3000),
+    (8, 32, 1024, 1024), (8, 32, 1025, 1025), (8, 31, 1024, 1024),
+])
+@pytest.mark.parametrize("op", ["positions", "chunk"])
+def test_positions_where_the_kernel_changes(op, n_kv, S, M, keys):
+    G.say(f"attention_{op} n_kv={n_kv} S={S} M={M}")
+    c = Call(op, keys - S, S, 82, n_kv, M)
+    got = c.alone()
+    kc, vc = (d.download(a.shape, np.uint16) for d, a in zip(c.dev, (c.kc, c.vc)))
+    Q = c.Q.copy()
+    if op == "chunk":
+        for t in range(S):
+            O.apply_rope(Q[t], c.K[t].copy(), c.start + t, TH, 4 * n_kv, n_kv, 128)
+    for t in sorted({0, 7, 8, S - 2, S - 1}):
+        exact = D.gqa_decode_f64(Q[t], kc, vc, 4 * n_kv, n_kv, 128, M, c.start + t)
+        D.check_close(got[t], exact, what=f"{op} n_kv={n_kv} S={S} M={M} t={t}")
+
+
+def test_few_rows_of_a_long_ring_use_the_device():
+    # 16 tokens of one kv head on a 64K ring: two row tiles, at most eight ranges
+    # of keys each, took 1.7 times as long as the decode kernel's 256 workgroups.
+    G.say("attention_positions n_kv=1, 16 tokens and 8 on a 64K ring")
+    ms = []
+    for S in (8, 16):
+        c = Call("positions", 65536 - S, S, 83, 1, 65536)
+        out = c.buffer()
+        ms.append(min(_call_ms(lambda: c(out, None), 20) for _ in range(3)))
+    print(f"{ms[0] * 1e3:.1f} us, {ms[1] * 1e3:.1f} us", flush=True)
+    assert ms[1] < 1.9 * ms[0]
