@@ -14,6 +14,7 @@
 
 #include "../../include/miattn.h"
 #include "../../include/mia_peaks.h"
+#include "mia_gemm_plan.h"
 #include "mia_kernels.h"
 
 // Scratch of mia_decode_step_noalloc, one copy per device for the life of the
@@ -854,10 +855,10 @@ int gemm_impl(DevCtx *c, int type, const void *W0, const void *W1, const void *W
 // Y [S][N] = X [S][K] . W^T for the K or V matrix of a layer (a type other than
 // Q4_0) from X's planes: [Xhi; Xlo] . Whi^T in one fp16 GEMM of 2S columns and,
 // for hi + lo weights, Xhi . Wlo^T in another, summed by the combine kernel.
-// The rings hold these sums rounded to fp16, so their rounding is kept as it
-// is: gemm_impl's sums are as close to the exact ones (3.0e-7 of a row against
-// 4.1e-7 here, 4096 values), but would move 0.3 % of the cached values to the
-// other fp16 neighbour.
+// The rings hold these sums rounded to fp16.  gemm_impl's sums are a little
+// closer to the exact ones (3.0e-7 of a row against 4.1e-7 here, 4096 values)
+// and put 0.3 % of the cached values on the other fp16 neighbour; so may another
+// process's choice of algorithm here (lt_gemm).
 int kv_projection(DevCtx *c, int type, const void *W, const _Float16 *planes, int N, int K, int S,
                   float *Y, hipStream_t s, bool packed) {
   const bool lo = gemm_two_planes(type);

@@ -220,10 +220,6 @@ struct GemmParams {
 // Q4_0 [N][K / 32] in the GGUF layout -> the GEMM tile layout (same size;
 // N and K multiples of 64, src 4-byte and dst 16-byte aligned, no overlap).
 hipError_t launch_q4_pack(const void *src, void *dst, int N, int K, hipStream_t s);
-// Sets tm and ksplit from N, K, S and the kind of weights.  plain: the K split
-// from N, K and S alone, by a fixed rule (sums that are rounded to fp16 and
-// kept, like a ring's keys and values, then do not move with the tuning).
-void gemm_plan(GemmParams &p, int num_cus, bool plain);
 hipError_t launch_gemm(const GemmParams &p, int mode, hipStream_t s, hipEvent_t ev0,
                        hipEvent_t ev1);
 // x [n] fp32 -> hi, lo [n] fp16 with x = hi + lo to ~2^-22 (n a multiple of 8).

@@ -25,6 +25,7 @@ import numpy as np
 import pytest
 
 import _data as D
+import _gemm_shapes as GS
 import _gpu as G
 import _oracle as O
 import anetransformers_amd as mia
@@ -270,10 +271,9 @@ def test_gemm_rows_of_every_magnitude(t):
     (O.TYPE_Q4_K, 14336, 4096), (O.TYPE_Q6_K, 4096, 14336),
 ])
 def test_gemm_f32_prefill_shapes_sampled(t, N, K):
-    # The Q4_K_M prefill layer's GEMMs at S = 512 (each shape's GEMM algorithm
-    # is picked on its first call): 64 sampled output columns against a
-    # float64 product of the oracle's dequantised rows, and a second call
-    # bit-identical to the first.
+    # The Q4_K_M prefill layer's GEMMs at S = 512: 64 sampled output columns
+    # against a float64 product of the oracle's dequantised rows, and a second
+    # call bit-identical to the first.
     S = 512
     G.say(f"kquant: gemm {NAMES[t]} S={S} {N}x{K}, sampled columns")
     g = np.random.default_rng(800 + N + K + t)
@@ -289,10 +289,8 @@ def test_gemm_f32_prefill_shapes_sampled(t, N, K):
 
 
 def test_gemm_f32_many_shapes():
-    # More GEMM shapes than the library remembers algorithms for (64): every
-    # batch size from 1 to 80 on one Q4_K and one Q6_K matrix, each against
-    # the oracle; the shapes past the limit run the heuristic's first
-    # algorithm untimed.
+    # Every batch size from 1 to 80 on one Q4_K and one Q6_K matrix, each
+    # against float64.
     G.say("kquant: gemm at 80 batch sizes x 2 types")
     g = np.random.default_rng(910)
     N, K = 96, 512
@@ -484,7 +482,7 @@ def test_prefill_layer_typed_all_q4_0_is_prefill_layer():
     (1, 328, 512),      # one token; 8 rows in the last workgroup's second wave
     (33, 264, 1024),    # one past the 32-token tile
     (65, 40, 2816),     # one past 64; fewer rows than a wave has; K split unevenly
-    (129, 520, 512),    # one past 128
+    (129, 520, 512),    # one past two 64-token tiles (128-token tiles: test_gemm_wide_token_tiles)
     (300, 4096, 512),   # unsplit, several tiles each way
 ])
 def test_gemm_tile_edges(t, S, N, K):
@@ -497,6 +495,86 @@ def test_gemm_tile_edges(t, S, N, K):
     got = gpu_gemm(W, t, X, N, K)
     Wd = O.dequant_typed(W, t, N, K).astype(np.float64)
     _assert_close(got, X.astype(np.float64) @ Wd.T, _bound(Wd, X), f"gemm edges {NAMES[t]}")
+
+
+KINDS = {"q4_k": O.TYPE_Q4_K, "f16": O.TYPE_F16, "q6_k": O.TYPE_Q6_K, "f32": O.TYPE_F32}
+
+
+@pytest.mark.parametrize("kind,S,N,K,split", GS.WIDE_GEMM)
+def test_gemm_wide_token_tiles(kind, S, N, K, split):
+    # 128-token tiles with a ragged last tile and ragged last weight rows, from
+    # the file's blocks against float64 within the row bound of fp32 sums, and
+    # from the packed form bit for bit the same
+    t = KINDS[kind]
+    G.say(f"gemm wide tiles {kind} S={S} {N}x{K}")
+    L = G.lib()
+    g = np.random.default_rng(11 * S + N + K + t)
+    W = O.make_typed(g, t, N, K, d_scale=0.07)
+    X = g.standard_normal((S, K)).astype(np.float32)
+    got = gpu_gemm(W, t, X, N, K)
+    Wd = O.dequant_typed(W, t, N, K).astype(np.float64)
+    _assert_close(got, X.astype(np.float64) @ Wd.T, _bound(Wd, X), f"gemm wide {kind}")
+    dp, dx, dy = gpu_pack(W, t, N, K), DB.from_array(X), DB(S * N * 4)
+    check(L.mia_gemm_packed_f32(dp.ptr, t, dx.ptr, dy.ptr, N, K, S, None), "packed gemm")
+    check(L.mia_stream_sync(None), "sync")
+    assert np.array_equal(dy.download((S, N), np.float32).view(np.uint32), got.view(np.uint32))
+
+
+@pytest.mark.parametrize("S,dim,hidden,split", GS.WIDE_LAYERS)
+def test_prefill_layer_wide_token_tiles(S, dim, hidden, split):
+    # the fused gate / up launch with 128-token tiles: the layer against the
+    # oracle at the bar of the other layers, and bit for bit the same packed
+    G.say(f"layer wide tiles S={S} dim={dim} hidden={hidden}")
+    L = G.lib()
+    nh, nkv, M, start, types = dim // 128, dim // 512, 512, 100, Q4_K_M
+    g = np.random.default_rng(S + hidden)
+    W = _layer(g, types, dim, hidden, nh, nkv)
+    kc, vc = D.ring(g, M, kv_dim=nkv * 128, filled=start)
+    X = g.standard_normal((S, dim)).astype(np.float32)
+    th = O.theta_inv(D.THETA, 128)
+    got, kc_g, vc_g = _run_layer(L, W, types, X, th, kc, vc, dim, hidden, nh, nkv, M, start, S)
+    ref = O.prefill_layer_typed(W, types, X, kc.copy(), vc.copy(), start, S, dim, hidden, nh, nkv, th)
+    assert np.abs(got - ref).max() <= 2e-3 * np.abs(ref).max()
+    kvd = nkv * 128
+    shapes = {"wq": (dim, dim), "wk": (kvd, dim), "wv": (kvd, dim), "wo": (dim, dim),
+              "w1": (hidden, dim), "w3": (hidden, dim), "w2": (dim, hidden)}
+    packs = {n: gpu_pack(W[n], types[n], *shapes[n]) for n in O.MATS}
+    norms = {n: DB.from_array(W[n]) for n in ("rms_att", "rms_ffn")}
+    lw = mia.LayerWeightsTyped(*[packs[n].ptr for n in O.MATS], *[types[n] for n in O.MATS],
+                               norms["rms_att"].ptr, norms["rms_ffn"].ptr)
+    dX, dth, dkc, dvc = DB.from_array(X), DB.from_array(th), DB.from_array(kc), DB.from_array(vc)
+    check(L.mia_prefill_layer_typed_packed(dX.ptr, ctypes.byref(lw), dth.ptr, dkc.ptr, dvc.ptr,
+                                           dim, hidden, nh, nkv, 1e-5, M, start, S, None),
+          "layer_typed_packed")
+    check(L.mia_stream_sync(None), "sync")
+    assert np.array_equal(dX.download(X.shape, np.float32).view(np.uint32), got.view(np.uint32))
+    assert np.array_equal(dkc.download(kc.shape, np.uint16), kc_g)
+    assert np.array_equal(dvc.download(vc.shape, np.uint16), vc_g)
+
+
+def test_prefill_layer_many_shapes():
+    # More GEMM shapes (90: 1 .. 60 and twice each) than the library remembers
+    # algorithms for in the K and V projections of layers (64): the cached rows
+    # of every batch size against float64, those past the limit with the
+    # heuristic's first algorithm, untimed.
+    G.say("layers at 60 batch sizes")
+    L = G.lib()
+    dim, hidden, nh, nkv, M, types = 512, 256, 4, 1, 64, Q4_K_M
+    g = np.random.default_rng(912)
+    W = _layer(g, types, dim, hidden, nh, nkv)
+    wv = O.dequant_typed(W["wv"], types["wv"], nkv * 128, dim).astype(np.float64)
+    th = O.theta_inv(D.THETA, 128)
+    kc, vc = D.ring(g, M, kv_dim=nkv * 128, filled=0)
+    for S in range(1, 61):
+        X = g.standard_normal((S, dim)).astype(np.float32)
+        _, _, vc_g = _run_layer(L, W, types, X, th, kc, vc, dim, hidden, nh, nkv, M, 0, S)
+        x = X.astype(np.float64)
+        xn = x / np.sqrt((x * x).mean(axis=1, keepdims=True) + 1e-5) * W["rms_att"]
+        want = xn @ wv.T
+        got = D.f16_bits_to_f32(vc_g[:S]).astype(np.float64)
+        # one fp16 rounding of a value that is good to fp32 sums
+        tol = 2.0 ** -11 * np.abs(want) + 2e-5 * np.abs(want).max(axis=1, keepdims=True)
+        assert np.all(np.abs(got - want) <= tol), S
 
 
 @pytest.mark.parametrize("t,K", [(O.TYPE_F16, 96), (O.TYPE_F32, 160), (O.TYPE_F16, 32)])

@@ -19,6 +19,7 @@ import numpy as np
 import pytest
 
 import _data as D
+import _gemm_shapes as GS
 import _gpu as G
 import _oracle as O
 import anetransformers_amd as mia
@@ -83,7 +84,7 @@ def test_gemm_more_tokens_than_a_grid_dimension():
     # more tokens than the second dimension of a launch may (65,535).  Token
     # rows repeat every 59, so every row must equal its first occurrence bit for
     # bit wherever it falls in the token tiles, and those match float64.
-    S, N, K, period = 66000, 32, 8192, 59
+    (S, N, K), period = GS.MANY_TOKENS, 59
     G.say(f"prefill: q4 gemm S={S} N={N} K={K}")
     L = G.lib()
     g = np.random.default_rng(66)
