@@ -12,29 +12,41 @@ namespace mia {
 constexpr int kGemmRows = 256;  // weight rows per workgroup
 
 // Sets tm and ksplit from N, K, S and the kind of weights.  plain: the K split
-// from N, K and S alone, by a fixed rule (sums that are rounded to fp16 and
-// kept, like a ring's keys and values, then do not move with the tuning).
+// by the fixed rule of ks_min alone (sums that are rounded to fp16 and kept, like
+// a ring's keys and values, then do not move with the tuning).
+//
 // 32, 64 or 128 tokens per workgroup, and the K split, by the time they are
-// expected to take (measured over S 8 .. 512 at 4096 / 5120 / 6144 / 28672 x
-// 4096 and 4096 x 14336; within 10 % of the best of all the choices there):
-//   - a 64-K stage takes a workgroup kAlone us while it has its CU to itself
-//     and kShared us of the CU's time when several share it (or follow each
-//     other);
-//   - a workgroup starts and ends in kEnds us (filling its stages, writing its
-//     tile), two of them at a time up to 64 tokens;
-//   - a K split adds the reduction: 4 us and reading the partial products at
-//     about 6 TB/s (they stay in the caches).
+// expected to take:
+//   - a 64-K stage takes a workgroup `alone` us, or `pair` us while another one is
+//     on its CU; a workgroup starts and ends in `ends` us (filling its stages,
+//     writing its tile);
+//   - with one workgroup to a CU (128 tokens; hi + lo weights) the workgroups run
+//     in whole rounds: 280 on 256 CUs take as long as 512.  Of pairs, a last round
+//     that is part empty costs `tail` of what is empty on top of its share;
+//   - a K split adds the reduction: 4.1 us and its partial products.
+// The figures are fitted to 864 shapes (S 2 .. 1024, 4096 for Q4_0; 4096 / 6144 /
+// 14336 / 28672 / 1024 x 4096, 4096 x 14336, 2048 x 1024, 512 x 2048, 8192 x 2560;
+// weights from HBM) at every tile and split.  Time over that of the best choice,
+// mean and worst, without whole rounds and here: Q4_0 1.013, 1.23 and 1.006,
+// 1.18; Q4_K 1.027, 1.31 and 1.002, 1.04; fp16 planes 1.036, 1.32 and 1.006,
+// 1.11; Q6_K 1.025, 1.24 and 1.000, 1.03; hi + lo planes 1.054, 1.33 and 1.007,
+// 1.18.
 // Splits stop where a workgroup would have fewer than four stages.  The split
 // does not depend on the form of the weights (Q4_0 in tiles or not, Q4_K or
 // its fp16 values, Q6_K or its planes), so that the sums are the same.
 inline void gemm_plan(GemmParams &p, int num_cus, bool plain) {
-  // [Q4_0, fp16 weights, hi + lo weights][32, 64, 128 tokens]
-  static const double kAlone[3][3] = {{0.62, 1.0, 0.0}, {0.85, 1.1, 1.88}, {1.8, 1.96, 3.0}};
-  static const double kShared[3][3] = {{0.56, 0.98, 0.0}, {0.85, 1.2, 1.88}, {1.6, 1.96, 3.0}};
-  static const double kEnds[3] = {1.5, 2.5, 5.0};
+  struct Cost {
+    double alone[3], pair[3], ends[3], tail;  // [32, 64, 128 tokens]; pair 0: one to a CU
+  };
+  static const Cost kCost[3] = {
+      {{0.511, 0.799, 0.0}, {0.906, 1.403, 0.0}, {1.8, 2.86, 0.0}, 0.103},  // Q4_0
+      {{0.53, 0.76, 1.17}, {1.36, 1.52, 0.0}, {3.3, 4.6, 8.6}, 0.25},  // fp16 weights
+      {{1.35, 1.9, 2.35}, {0.0, 0.0, 0.0}, {2.7, 4.9, 15.0}, 0.0},     // hi + lo weights
+  };
   const int kind = p.src == kGemmQ40Tile || p.src == kGemmQ40 ? 0
                    : p.src == kGemmQ4K || p.src == kGemmF16   ? 1
                                                               : 2;
+  const Cost &c = kCost[kind];
   const long n_all = p.K / gemm_k_unit(p.K);
   // A sum's rounding grows with its length: up to this many splits, partial
   // sums are kept short wherever 64-token tiles leave the device unfilled.
@@ -48,12 +60,15 @@ inline void gemm_plan(GemmParams &p, int num_cus, bool plain) {
     for (int ks = ks_min; ks <= (plain ? ks_min : 16); ks *= 2) {
       if (ks > ks_min && n_all / ks < 4) break;
       const double wgs = (double)(tiles * ks) / num_cus;  // per CU
-      const double share = wgs <= 2.0 ? std::ceil(wgs) : wgs + 0.25;
-      const double stage =
-          share <= 1.0 ? kAlone[kind][i] : std::max(kAlone[kind][i], kShared[kind][i] * share);
-      double us = stage * (double)((n_all + ks - 1) / ks) +
-                  kEnds[i] * std::ceil(i < 2 ? share / 2 : share);
-      if (ks > 1) us += 4.0 + 4e-6 / 6.0 * (double)ks * p.S * p.N;
+      const double stages = (double)((n_all + ks - 1) / ks);
+      double us = c.alone[i] * stages + c.ends[i];
+      if (wgs > 1.0 && c.pair[i] == 0.0) {
+        us *= std::ceil(wgs);
+      } else if (wgs > 1.0) {
+        const double pairs = std::max(1.0, wgs / 2);
+        us = (pairs + c.tail * (std::ceil(pairs) - pairs)) * (c.pair[i] * stages + c.ends[i]);
+      }
+      if (ks > 1) us += 4.1 + 1.2e-6 * (double)ks * p.S * p.N;
       if (best == 0.0 || us < best) {
         best = us;
         p.tm = 1 << i;
@@ -61,6 +76,9 @@ inline void gemm_plan(GemmParams &p, int num_cus, bool plain) {
       }
     }
   }
+  // hi + lo planes of few tokens are bound by their 4 bytes a weight, which 32-token
+  // tiles in two rounds read faster (14336 x 4096, 33 tokens: 63 us, 80 in one round)
+  if (p.src == kGemmF16x2 && p.S <= 64 && p.ksplit <= 4) p.tm = 1;
 }
 
 }  // namespace mia

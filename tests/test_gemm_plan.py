@@ -59,4 +59,23 @@ def test_wide_layer_shapes(plan, S, dim, hidden, split):
 def test_split_of_many_tokens(plan):
     # the shape by which the GPU tests have a K split of more than 65,535 tokens
     S, N, K = GS.MANY_TOKENS
-    assert S > 65535 and plan(Q40, S, N, K)[1] > 1
+    assert S > 65535 and plan(Q6K, S, N, K)[1] > 1
+
+
+@pytest.mark.parametrize("src,S,N,K,slow", [
+    # choices that had cost 13 to 40 % more than another: a last round of a few
+    # workgroups, and splits of weights that memory bounds
+    (Q40_TILE, 777, 4096, 4096, (1, 2)), (Q4K, 777, 14336, 4096, (4, 2)),
+    (F16, 777, 6144, 4096, (4, 4)), (F16X2, 33, 14336, 4096, (2, 4)),
+    (F16X2, 300, 4096, 4096, (2, 8)), (Q4K, 64, 4096, 4096, (2, 16)),
+])
+def test_plan_avoids_slow_choices(plan, src, S, N, K, slow):
+    assert plan(src, S, N, K) != slow
+
+
+@pytest.mark.parametrize("kind", ["q4_0", "q4_k", "q6_k"])
+def test_split_is_the_same_in_both_forms(plan, kind):
+    a, b = SOURCES[kind]
+    for N, K in ((4096, 4096), (14336, 4096), (4096, 14336), (1024, 4096), (520, 2048), (96, 512)):
+        for S in (1, 8, 33, 64, 65, 100, 129, 300, 444, 512, 777, 1024, 2048, 5000):
+            assert plan(a, S, N, K)[1] == plan(b, S, N, K)[1]

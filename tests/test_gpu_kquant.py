@@ -520,6 +520,29 @@ def test_gemm_wide_token_tiles(kind, S, N, K, split):
     assert np.array_equal(dy.download((S, N), np.float32).view(np.uint32), got.view(np.uint32))
 
 
+def test_gemm_more_tokens_than_a_grid_dimension():
+    # 66,000 tokens with the K range split in two: the sum of the splits covers
+    # more tokens than the second dimension of a launch may (65,535).  Token
+    # rows repeat every 59, so every row must equal its first occurrence bit for
+    # bit wherever it falls in the token tiles, and those match float64.
+    (S, N, K), period, t = GS.MANY_TOKENS, 59, O.TYPE_Q6_K
+    G.say(f"kquant: gemm {NAMES[t]} S={S} {N}x{K}")
+    L = G.lib()
+    g = np.random.default_rng(66)
+    W = O.make_typed(g, t, N, K, d_scale=0.07)
+    base = g.standard_normal((period, K)).astype(np.float32)
+    dw, dx, dy = DB.from_array(W), DB(S * K * 4), DB(S * N * 4)
+    rows = np.tile(base, (20, 1))
+    for s in range(0, S, len(rows)):
+        dx.upload(rows[:S - s], offset=s * K * 4)
+    check(L.mia_gemm_f32(dw.ptr, t, dx.ptr, dy.ptr, N, K, S, None), "gemm")
+    check(L.mia_stream_sync(None), "sync")
+    got = dy.download((S, N), np.float32)
+    Wd = O.dequant_typed(W, t, N, K).astype(np.float64)
+    _assert_close(got[:period], base.astype(np.float64) @ Wd.T, _bound(Wd, base), "gemm many tokens")
+    assert np.array_equal(got, got[np.arange(S) % period])
+
+
 @pytest.mark.parametrize("S,dim,hidden,split", GS.WIDE_LAYERS)
 def test_prefill_layer_wide_token_tiles(S, dim, hidden, split):
     # the fused gate / up launch with 128-token tiles: the layer against the

@@ -19,7 +19,6 @@ import numpy as np
 import pytest
 
 import _data as D
-import _gemm_shapes as GS
 import _gpu as G
 import _oracle as O
 import anetransformers_amd as mia
@@ -77,30 +76,6 @@ def test_gemm_matches_oracle(S, out_dim, in_dim):
     err = np.abs(got.astype(np.float64) - ref)
     assert np.all(err <= bound), float((err / bound).max())
     D.check_close(got, ref, what=f"gemm {S}x{out_dim}x{in_dim}")
-
-
-def test_gemm_more_tokens_than_a_grid_dimension():
-    # 66,000 tokens with the K range split in two: the sum of the splits covers
-    # more tokens than the second dimension of a launch may (65,535).  Token
-    # rows repeat every 59, so every row must equal its first occurrence bit for
-    # bit wherever it falls in the token tiles, and those match float64.
-    (S, N, K), period = GS.MANY_TOKENS, 59
-    G.say(f"prefill: q4 gemm S={S} N={N} K={K}")
-    L = G.lib()
-    g = np.random.default_rng(66)
-    W = O.make_q4_0(g, N, K)
-    base = g.standard_normal((period, K)).astype(np.float32)
-    dw, dx, dy = DB.from_array(W), DB(S * K * 4), DB(S * N * 4)
-    chunk = np.tile(base, (20, 1))
-    for t in range(0, S, len(chunk)):
-        dx.upload(chunk[:S - t], offset=t * K * 4)
-    check(L.mia_q4_0_gemm_f32(dw.ptr, dx.ptr, dy.ptr, N, K, S, None), "gemm")
-    check(L.mia_stream_sync(None), "sync")
-    got = dy.download((S, N), np.float32)
-    Wd = O.dequant_q4_0(W, N, K).astype(np.float64)
-    bound = 2 * K * 2.0 ** -24 * (np.abs(base.astype(np.float64)) @ np.abs(Wd).T) + K * 6e-8 * np.abs(Wd).max()
-    assert np.all(np.abs(got[:period] - base.astype(np.float64) @ Wd.T) <= bound)
-    assert np.array_equal(got, got[np.arange(S) % period])
 
 
 def _layer(g, dim, hidden, nh, nkv):
