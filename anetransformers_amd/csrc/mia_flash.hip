@@ -1792,11 +1792,20 @@ size_t flash_scratch_bytes(int n_kv, int n_rtiles, int nsplit, int rows_per_tile
 // Few rows (S*G <= 32, e.g. speculative verify): one 32-row block, key splits
 // over workgroups until about target_wgs workgroups.  Otherwise (prefill):
 // 64-row tiles, no split unless the row tiles alone leave the device mostly
-// idle.  Every wave of a split keeps at least one tile of 32 keys, and ranges of
-// fewer than four such splits stay whole (eight drafts after 250 keys, two
-// splits: 56 against 50 us for four layers; after 1000 keys, seven splits: 56.5
-// against 69.8 unsplit, and 65.1 with at least two tiles a wave).
-// Without staged rows keys are slots (flash_kernel).
+// idle.  Every wave of a split keeps at least one tile of 32 keys, and a range is
+// split only where that saves more than the merge takes, a launch with a
+// workgroup per row.  Us a step with drafts on a wrapped ring, 8 kv heads, whole
+// and split (a range of 1000 keys takes a 32-row tile 8.8 us, a 64-row tile
+// 10.8):
+//   drafts   512 keys     600          850          1000         1300         2100
+//        8   15.2  14.6   15.5  14.6   16.3  14.7   17.4  13.8   20.5  15.3   26.3  16.4
+//       16   20.0  18.0   19.9  18.0   21.6  17.7   22.6  17.5   28.0  18.5   36.3  19.8
+//       33   20.2  22.1   20.8  22.4   22.9  22.2   24.3  21.9   30.3  23.4   40.5  24.3
+//       64   20.4  25.4   20.2  25.6   22.5  26.2   23.0  26.9   29.2  27.7   36.9  28.6
+//      100   20.8  32.3   21.1  32.3   23.9  32.7   24.7  32.1   29.9  34.5   38.7  37.4
+//      200   21.5  44.6   22.6  46.7   24.4  49.0   25.8  47.8   31.8  50.8   42.3  55.9
+// Without staged rows (8 queries: 9.2 and 10.1 us at 512 keys, 12.9 and 11.0 at
+// 1000) keys are slots (flash_kernel).
 void flash_plan(int S, int n_kv, int G, int start_pos, int max_seq, bool staged, int target_wgs,
                 int *n_rtiles, int *nsplit, int *split_keys, int *rows_per_tile_out) {
   const int rt = rows_per_tile(S);
@@ -1815,13 +1824,18 @@ void flash_plan(int S, int n_kv, int G, int start_pos, int max_seq, bool staged,
   long want = (long)target_wgs / ((long)n_kv * ntiles);
   if (want < 1) want = 1;
   long max_split = maxkeys / (kWaves * kKT);
-  if (max_split < 4) max_split = 1;
   if (max_split > kMergeSplitsPerThread * 32) max_split = kMergeSplitsPerThread * 32;
   if (want > max_split) want = max_split > 0 ? max_split : 1;
   long sk = (maxkeys + want - 1) / want;
   sk = ((sk + kKT - 1) / kKT) * kKT;
   long ns = (maxkeys + sk - 1) / sk;
   if (ns < 1) ns = 1;
+  const double saved = 1e-3 * (rt == 32 ? 8.8 : 10.8) * maxkeys * (1.0 - 1.0 / ns);
+  const double merge = (staged ? 1.4 : 3.7) + 4.2e-3 * n_kv * ntiles * rt;
+  if (saved < merge) {
+    ns = 1;
+    sk = (maxkeys + kKT - 1) / kKT * kKT;
+  }
   *n_rtiles = ntiles;
   *nsplit = (int)ns;
   *split_keys = (int)sk;

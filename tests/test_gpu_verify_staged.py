@@ -25,6 +25,7 @@ import _oracle as O
 import anetransformers_amd as mia
 from anetransformers_amd import DeviceBuffer as DB
 from anetransformers_amd import check
+from test_gpu_positions import _call_ms
 
 pytestmark = pytest.mark.gpu
 
@@ -73,6 +74,46 @@ def test_staged_step_matches_sequential_and_leaves_ring(M, start, S):
     # and bit for bit what the writing form of the step puts in the ring
     _, kc_w, vc_w = G.attention_step(kc, vc, Q, K, V, TH, M, start, S)
     assert np.array_equal(kc_w[pos % M], ks) and np.array_equal(vc_w[pos % M], vs)
+
+
+@pytest.mark.parametrize("M,S", [(480, 8), (512, 8), (450, 16), (512, 16), (700, 33), (900, 33),
+                                 (1000, 64), (1300, 64), (600, 200)])
+def test_staged_step_whole_and_split(M, S):
+    # Both sides of where the keys are split and merged, against float64.
+    G.say(f"staged step whole or split M={M} S={S}")
+    g = D.rng(11 * M + S)
+    start = M + 77
+    kc, vc = D.ring(g, M)
+    Q, K, V = D.normal(g, (S, 4096)), D.normal(g, (S, D.KV_DIM)), D.normal(g, (S, D.KV_DIM))
+    out, _, _, ks, vs = staged(kc, vc, Q, K, V, M, start, S)
+    for t in range(S):
+        O.apply_rope(Q[t], K[t].copy(), start + t, TH, 32, 8, 128)
+        kc[(start + t) % M], vc[(start + t) % M] = ks[t], vs[t]  # (the ring as query t sees it)
+        if t in (0, 1, 7, 8, S // 2, S - 1):
+            exact = D.gqa_decode_f64(Q[t], kc, vc, 32, 8, 128, M, start + t)
+            D.check_close(out[t], exact, what=f"M={M} S={S} t={t}")
+
+
+def test_a_split_that_does_not_pay_is_not_made():
+    # 200 drafts on a ring of 600: two ranges of 300 keys saved 3 us and took 24
+    # to merge, and 300 drafts, which fill the device unsplit, took half the time.
+    G.say("staged steps of 200 and 300 drafts, ring of 600")
+    L, M = G.lib(), 600
+    ms = []
+    for S in (200, 300):
+        g = D.rng(S)
+        kc, vc = D.ring(g, M)
+        b = [DB.from_array(a) for a in (D.normal(g, (S, 4096)), D.normal(g, (S, D.KV_DIM)),
+                                        D.normal(g, (S, D.KV_DIM)), TH, kc, vc)]
+        ks, vs, out = DB(S * ROW), DB(S * ROW), DB(S * 4096 * 4)
+
+        def step():
+            check(L.mia_attention_step_staged(*(x.ptr for x in b), ks.ptr, vs.ptr, out.ptr, 32, 8,
+                                              128, M, M + 1000, S, None), "staged")
+
+        ms.append(min(_call_ms(step, 20) for _ in range(3)))
+    print(f"{ms[0] * 1e3:.1f} us, {ms[1] * 1e3:.1f} us", flush=True)
+    assert ms[0] < 1.4 * ms[1]
 
 
 def test_commit_keeps_only_accepted_rows_across_layers():
