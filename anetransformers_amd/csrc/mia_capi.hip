@@ -67,17 +67,20 @@ bool few_positions(int S, int n_kv, int max_seq, int num_cus) {
 // step, 64-row tiles with the merge as a launch of its own, then here (tiles:
 // kv heads x tokens / 8):
 //   tiles   256 keys     800          1024         2048         4096         8192
-//       3   10.0   8.0   13.3  12.9   12.9  14.2   12.8  16.0   12.9  18.2   14.0  20.4
-//      16   10.4   8.0   14.0  12.5   13.7  13.4   14.5  14.6   17.7  18.2   18.0  21.7
-//      24   10.3   7.9   16.0  12.5   16.5  13.3   17.6  16.0   17.1  18.1   19.6  21.5
-//      32   10.2   8.2   16.1  12.4   16.8  13.4   19.1  17.5   19.8  18.8   21.3  23.6
-//      64   10.6   8.3   21.7  12.8   22.9  13.5   23.6  17.2   26.2  20.8   30.9  29.2
-//     128   10.8   8.6   30.7  12.9   31.0  14.0   33.7  19.9   39.9  28.3   51.5  45.8
-//     256   10.9   8.6   47.7  13.7   48.3  14.8   54.0  24.4   67.3  41.4   93.9  76.9
-// 128 tiles: 65.3 and 62.6 at 12,288 keys, 79.2 and 80.4 at 16,384, 250 and 300 at
-// 65,536; 3 tiles there: 21.0 and 78.0.
+//       3   10.1   7.8   13.1  12.8   12.6  14.1   12.8  16.1   13.1  18.1   14.1  20.5
+//      16   10.1   8.0   13.6  12.6   13.6  13.4   14.9  16.1   17.6  18.3   17.8  21.7
+//      24   10.2   7.9   17.5  12.5   16.4  13.4   17.8  16.2   18.5  18.6   20.6  22.2
+//      32   10.2   7.9   16.7  12.4   16.7  13.5   19.2  16.2   19.8  19.0   21.4  23.7
+//      40   10.3   8.1   17.5  12.6   19.4  13.7   20.2  16.4   23.3  19.6   27.0  25.9
+//      64   10.3   8.1   16.8  12.4   17.9  13.6   23.2  16.9   25.8  20.6   30.4  29.6
+//     128   10.3   8.3   16.8  12.6   18.3  14.1   28.1  20.2   39.9  29.5   51.5  45.5
+//     256   10.6   8.4   17.3  13.4   18.5  15.9   28.6  23.6   49.5  41.3   93.5  76.9
+// At 12,288 keys 64 tiles 37.6 and 37.9, 96 tiles 52.6 and 55.1, 128 tiles 65.2 and
+// 63.1; at 16,384 128 tiles 79.4 and 80.1; at 65,536 250 and 300, 3 tiles 21.0 and
+// 78.0.
 bool shared_tiles_pay(long tiles, long keys) {
-  return keys <= 900 || (keys <= 12288 && keys <= (tiles < 20 ? 64 : 160) * tiles);
+  if (keys <= 900) return true;
+  return keys <= (tiles < 20 ? 64 : 200) * tiles && keys <= (tiles < 128 ? 9216 : 12288);
 }
 // The K and V projections of layers of other weight types (hipBLASLt): workspace
 // size, algorithms timed on a shape's first call, shapes remembered.

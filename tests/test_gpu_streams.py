@@ -192,8 +192,9 @@ def test_fewer_kv_heads(op, n_kv, S):
 @pytest.mark.parametrize("n_kv,S,M,keys", [
     (1, 17, 4096, 900), (1, 17, 4096, 901),      # short windows: tiles that share keys at any count
     (8, 16, 4096, 1024), (8, 16, 4096, 1025),    # 16 tiles
-    (8, 24, 4096, 3840), (8, 24, 4096, 3841),    # 24 tiles
-    (8, 80, 16384, 12288), (8, 80, 16384, 12289),
+    (8, 24, 8192, 4800), (8, 24, 8192, 4801),    # 24 tiles
+    (8, 80, 16384, 9216), (8, 80, 16384, 9217),
+    (8, 128, 16384, 12288), (8, 128, 16384, 12289),
 ])
 def test_batch_where_the_kernel_changes(n_kv, S, M, keys):
     G.say(f"attention_batch n_kv={n_kv} S={S} keys={keys}")
