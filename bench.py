@@ -1100,12 +1100,14 @@ def load_traffic(name: str):
     try:
         with open(path) as f:
             entry = json.load(f).get(name)
-        src = os.path.join(REPO, entry["kernel_source"])
-        with open(src, "rb") as f:
-            if hashlib.sha256(f.read()).hexdigest() != entry["kernel_source_sha256"]:
-                log(f"roofline.traffic for {name}: {entry['kernel_source']} changed since its "
-                    "counters were measured; reported as null")
-                return None
+        sha = hashlib.sha256()
+        for src in entry["kernel_source"].split():  # the files that hold the kernel
+            with open(os.path.join(REPO, src), "rb") as f:
+                sha.update(f.read())
+        if sha.hexdigest() != entry["kernel_source_sha256"]:
+            log(f"roofline.traffic for {name}: {entry['kernel_source']} changed since its "
+                "counters were measured; reported as null")
+            return None
         return int(entry["bytes"])
     except (OSError, ValueError, KeyError, TypeError):
         return None

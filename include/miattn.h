@@ -139,7 +139,11 @@ int mia_decode_step_noalloc(const float *q, const float *k, const float *v,
 
 /* S>=1 causal GQA attention over the ring as it stands, query t at position
  * start_pos + t.  Replaces attention_batch (mistral/mistral_ane_prefill.h:
- * 207-275).  Q [S][n_heads*128] fp32 dev, rotated; out [S][n_heads*128]. */
+ * 207-275).  Q [S][n_heads*128] fp32 dev, rotated; out [S][n_heads*128].
+ * A value that is not finite in a row of the batch's own positions may also
+ * spoil the outputs of up to 15 queries before it (a key past a query's
+ * position has weight 0 there); so in mia_attention_step with S > 1.
+ * mia_attention_positions and mia_attention_chunk keep a query to its window. */
 int mia_attention_batch(const float *Q, float *out, const uint16_t *k_layer,
                         const uint16_t *v_layer, int n_heads, int n_kv_heads, int hd,
                         int max_seq, int start_pos, int S, void *stream);
